@@ -136,6 +136,29 @@ def test_correction_collisions_and_reuse(dev):
     ws.close()
 
 
+@pytest.mark.parametrize("count", [0, 1, 63, 255, 256, 257, 600])
+@pytest.mark.parametrize("dim", [2, 3])
+def test_correction_event_regions(dev, dim, count):
+    """Every particle escaped and every corner inside, at counts around a
+    block of particles, in a workspace of exactly that many events: each
+    block's region of events is full, the last one partly there.  Bit-exact
+    (max and min of one rounded value per corner)."""
+    n = 16
+    win = D.GridWindow((0, 0, 0), (n, n, n if dim == 3 else 1), (0.1, 0.1, 0.1))
+    phi = np.full(win.shape, 2.0)
+    rng = np.random.default_rng(count + dim)
+    P = np.zeros((count, 4))
+    P[:, :dim] = 1 + (n - 3) * rng.random((count, dim))
+    P[:, 3] = -rng.uniform(0.1, 0.5, count)
+    ws = PL.CorrectionWorkspace(win.nodes, max(count, 1) * 2 ** dim)
+    ref = O.pls_correct(P, phi, owin(win), None, 0, dim)
+    for _ in range(2):                                 # the workspace is neutral again after a call
+        pd = to_dev(phi)
+        PL.correct(to_dev(P), pd, win, ws)
+        assert np.array_equal(to_np(pd), ref)
+    ws.close()
+
+
 @pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
 @pytest.mark.parametrize("dim", [2, 3])
 def test_adjust_radii(dev, dtype, dim):
