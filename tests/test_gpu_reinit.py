@@ -85,6 +85,24 @@ def test_reinit_batch(dev):
         _check(phi, win, recs, dphi, band)
 
 
+@pytest.mark.parametrize("n", [(112, 112, 112), (128, 7, 24), (9, 61, 4), (301, 9, 1), (6, 5, 1), (7, 1, 9)])
+def test_reinit_heap_levels_and_faces(dev, n):
+    """A sphere whose heap is deeper than the part of it in LDS, and windows
+    so thin that every node's stencil leaves them."""
+    win = D.GridWindow((-3, 4, 1 if n[2] > 1 else 0), n, (1.0, 1.0, 1.0))
+    if min(n) > 100:
+        phi = _sphere(n[0], (55.3, 54.6, 56.2), 40.4, 1.7)
+    else:
+        z, y, x = np.meshgrid(*(np.arange(float(k)) for k in n[::-1]), indexing="ij")
+        phi = 1.7 * (0.8 * (x - 0.47 * n[0]) + 0.5 * (y - 0.4 * n[1]) + 0.3 * (z - 0.6 * n[2]))
+        phi = phi if n[2] > 1 else phi[0]
+    phi = np.ascontiguousarray(phi)
+    recs, drecs = _case(phi, win)
+    dphi = to_dev(phi)
+    (band,) = M.reinitialize([(dphi, win, drecs, len(recs))])
+    _check(phi, win, recs, dphi, band)
+
+
 def test_reinit_empty_and_heap_error(dev):
     n = 20
     win = D.GridWindow((0, 0, 0), (n, n, n), (1.0, 1.0, 1.0))
