@@ -10,7 +10,8 @@
 // or LDS-ring columns) and the resident blocks per CU come from a table of
 // configurations, and the ring columns' z-chunk is chosen per cell-size
 // class; dcl_batch_autotune times them on the caller's buffers and keeps the
-// fastest.  2D cells: 64 x 4 node tiles, one node per thread.  Band mode
+// fastest.  2D cells: SL and curvature of a tile in one pass (dcl_step2d.hpp),
+// one launch.  Band mode
 // (dcl_batch_band_step): only the listed nodes of every cell, as the
 // reference's band loop (LevelSetMethod/AdvectSL.c:23-89), one thread per
 // node over the packed band list.
@@ -23,6 +24,7 @@
 
 #include "dcl_host.hpp"
 #include "dcl_ring.hpp"
+#include "dcl_step2d.hpp"
 #include "dcl_tile.hpp"
 
 namespace dcl {
@@ -57,8 +59,8 @@ __host__ __device__ constexpr TileShape shape_of(int s) {
 }
 constexpr int NOCC = 3;
 constexpr int occ_of(int o) { return o == 0 ? 2 : o == 1 ? 4 : 8; }  // resident blocks per CU
-// 2D tiles: 64 x 4 nodes
-constexpr int T2X = 64, T2Y = 4;
+// 2D tiles: 62 x 14 nodes of 64 x 16 worked, four rows per thread
+constexpr int T2R = 4, T2X = Step2<T2R>::OX, T2Y = Step2<T2R>::OY;
 // cell-size classes (largest axis up to 48, up to 80, beyond) and the ring
 // z-chunks tried for each
 constexpr int NCLASS = DCL_BATCH_CLASSES;
@@ -86,29 +88,35 @@ struct WorkQ {
 
 template <typename F>
 __device__ __forceinline__ void claim_tiles(WorkQ* __restrict__ q, const int* __restrict__ bounds, int k, F body) {
-  const int xcd = blockIdx.x & 7;
-  if (k <= 0) {
-    const int nslot = gridDim.x >> 3, slot = blockIdx.x >> 3;
-    for (int t = bounds[xcd] + slot; t < bounds[xcd + 1]; t += nslot) body(t);
-    return;
-  }
   __shared__ int s_tile;
+  const int xcd = blockIdx.x & 7;
   const bool lead = threadIdx.x == 0 && threadIdx.y == 0;
-  for (int s = 0; s < 8; ++s) {
-    const int x = (xcd + s) & 7;
-    const int lo = bounds[x], hi = bounds[x + 1];
-    if (lo >= hi) continue;
-    for (;;) {
-      if (lead) s_tile = lo + k * (int)atomicAdd(&q->claim[x], 1u);
-      __syncthreads();
-      const int t0 = s_tile;
-      __syncthreads();
-      if (t0 >= hi) break;
-      const int t1 = min(t0 + k, hi);
-      for (int t = t0; t < t1; ++t) body(t);
-    }
+  // tiles t, t + step, ... below t1, then the next claim (body is inlined once)
+  int t = 0, t1 = 0, step = 1, s = 0;
+  if (k <= 0) {
+    t = bounds[xcd] + (int)(blockIdx.x >> 3);
+    t1 = bounds[xcd + 1];
+    step = (int)(gridDim.x >> 3);
   }
-  if (lead && atomicAdd(&q->done, 1u) == gridDim.x - 1) {
+  for (;; t += step) {
+    if (t >= t1) {
+      if (k <= 0) break;
+      for (; s < 8; ++s) {
+        const int x = (xcd + s) & 7;
+        const int lo = bounds[x], hi = bounds[x + 1];
+        if (lo >= hi) continue;
+        if (lead) s_tile = lo + k * (int)atomicAdd(&q->claim[x], 1u);
+        __syncthreads();
+        t = s_tile;
+        __syncthreads();
+        t1 = min(t + k, hi);
+        if (t < hi) break;
+      }
+      if (s == 8) break;
+    }
+    body(t);
+  }
+  if (k > 0 && lead && atomicAdd(&q->done, 1u) == gridDim.x - 1) {
     for (int x = 0; x < 8; ++x) atomicExch(&q->claim[x], 0u);
     atomicExch(&q->done, 0u);
   }
@@ -196,28 +204,21 @@ __global__ __launch_bounds__(shape_of(S).tx * shape_of(S).ty) void batch_curv_k(
   });
 }
 
-// 2D cells: one node per thread over 64 x 4 tiles; nodes outside [2, n-3]
-// copy phi0 (as the dense 2D step)
+// 2D cells: SL and curvature of one tile after another (nodes outside
+// [2, n-3] copy phi0, as in the dense 2D step)
 template <typename T, int INTERP, int BT>
-__global__ __launch_bounds__(T2X * T2Y) void batch2d_sl_k(const T* __restrict__ phi0, T* __restrict__ phi,
-                                                         const T* __restrict__ vel, const BCell* __restrict__ cells,
-                                                         const int4* __restrict__ tiles,
-                                                         const int* __restrict__ bounds, WorkQ* __restrict__ q, int k) {
+__global__ __launch_bounds__(Step2<T2R>::NT) void batch2d_step_k(const T* __restrict__ phi0, T* __restrict__ phi,
+                                                                 T* __restrict__ kappa, const T* __restrict__ vel,
+                                                                 const BCell* __restrict__ cells,
+                                                                 const int4* __restrict__ tiles,
+                                                                 const int* __restrict__ bounds,
+                                                                 WorkQ* __restrict__ q, int k) {
+  __shared__ Step2Lds<T, T2R> S;
   claim_tiles(q, bounds, k, [&](int t) {
     const int4 tl = tiles[t];
     const BCell c = cells[tl.x];
-    const int i = tl.y + threadIdx.x, j = tl.z + threadIdx.y;
-    if (i < c.nx && j < c.ny) {
-      const SLP P = cell_slp<2>(c);
-      const int id = j * c.nx + i;
-      const T* p0 = phi0 + c.phi_off;
-      T v;
-      if (i >= 2 && i <= c.nx - 3 && j >= 2 && j <= c.ny - 3)
-        v = sl_point<T, 2, INTERP, BT>(p0, vel + c.vel_off, P, c.px + i, c.py + j, c.pz);
-      else
-        v = p0[id];
-      phi[c.phi_off + id] = v;
-    }
+    step2d_tile<T, INTERP, BT, T2R>(phi0 + c.phi_off, phi + c.phi_off, kappa + c.phi_off, vel + c.vel_off,
+                                    cell_slp<2>(c), curv_recips<T>(c.dx, c.dy, 1.0), tl.y, tl.z, S);
   });
 }
 
@@ -227,19 +228,6 @@ template <typename T>
 __device__ __forceinline__ T curv2d_node(const T* __restrict__ p, const BCell& c, int i, int j) {
   if (i < 1 || i > c.nx - 2 || j < 1 || j > c.ny - 2) return T(0);
   return curv2d_at<T>(p + j * c.nx + i, c.nx, (T)c.dx, (T)c.dy);
-}
-
-template <typename T>
-__global__ __launch_bounds__(T2X * T2Y) void batch2d_curv_k(const T* __restrict__ phi, T* __restrict__ kappa,
-                                                           const BCell* __restrict__ cells,
-                                                           const int4* __restrict__ tiles,
-                                                           const int* __restrict__ bounds, WorkQ* __restrict__ q, int k) {
-  claim_tiles(q, bounds, k, [&](int t) {
-    const int4 tl = tiles[t];
-    const BCell c = cells[tl.x];
-    const int i = tl.y + threadIdx.x, j = tl.z + threadIdx.y;
-    if (i < c.nx && j < c.ny) kappa[c.phi_off + j * c.nx + i] = curv2d_node<T>(phi + c.phi_off, c, i, j);
-  });
 }
 
 // Band mode: entry b of the packed list is {x, y, z, cell} in the cell's
@@ -297,7 +285,7 @@ struct KTable {
     }
   }
   static const void* ring() { return (const void*)&batch_ring_k<T, INTERP, BT>; }
-  static const void* sl2d() { return (const void*)&batch2d_sl_k<T, INTERP, BT>; }
+  static const void* step2d() { return (const void*)&batch2d_step_k<T, INTERP, BT>; }
   static const void* band(int dim) {
     return dim == 3 ? (const void*)&batch_band_sl_k<T, 3, INTERP, BT>
                     : (const void*)&batch_band_sl_k<T, 2, INTERP, BT>;
@@ -317,10 +305,10 @@ static const void* curv_kernel(int s) {
 }
 
 // SL kernels by kind: 0 tile gathers of shape s, 1 ring columns, 2 2D
-// tiles, 3 band mode of dimension s
+// tiles (the curvature with them), 3 band mode of dimension s
 template <typename K>
 static const void* sl_pick(int kind, int s) {
-  return kind == 0 ? K::sl(s) : kind == 1 ? K::ring() : kind == 2 ? K::sl2d() : K::band(s);
+  return kind == 0 ? K::sl(s) : kind == 1 ? K::ring() : kind == 2 ? K::step2d() : K::band(s);
 }
 
 template <typename T>
@@ -366,7 +354,7 @@ static int upload_cells(dcl_batch b) {
   return 0;
 }
 
-// tile list s < NBASE: tiles of shape s (2D batches: s = 0, 64 x 4 tiles);
+// tile list s < NBASE: tiles of shape s (2D batches: s = 0, the 2D tiles);
 // s == RING_LIST: 32 x 8 columns of each cell's z-chunk.  Cells come largest
 // first (a block that claims late gets a small tile), each cell's tiles in
 // raster order; the list is cut into 8 contiguous chunks of about equal cost,
@@ -438,7 +426,8 @@ static int grid_blocks(dcl_batch b, int occ) {
   return g < 8 ? 8 : g - g % 8;
 }
 
-// the two launches of one step with configuration (s, occ)
+// the two launches of one step with configuration (s, occ); 2D: one (kcv is
+// NULL)
 struct Plan {
   const void* ksl;
   const void* kcv;
@@ -460,11 +449,11 @@ static int make_plan(dcl_batch b, int s, int occ, Plan& p) {
   p.qcv = b->queues + 1;
   if (b->dim == 2) {
     DCL_TRY(build_tiles(b, 0));
-    p.bsl = p.bcv = dim3(T2X, T2Y);
+    p.bsl = p.bcv = dim3(S2_TX, S2_TY);
     p.tsl = p.tcv = b->tiles[0];
     p.bsl_bounds = p.bcv_bounds = b->bounds[0];
     p.ksl = f64 ? sl_kernel<double>(b->interp, b->backtrace, 2, 0) : sl_kernel<float>(b->interp, b->backtrace, 2, 0);
-    p.kcv = f64 ? (const void*)&batch2d_curv_k<double> : (const void*)&batch2d_curv_k<float>;
+    p.kcv = nullptr;
     return 0;
   }
   const int cs = s % NBASE;
@@ -491,19 +480,40 @@ static int make_plan(dcl_batch b, int s, int occ, Plan& p) {
   return 0;
 }
 
+// the arguments of a plan's launches (pointers to the members)
+struct PlanArgs {
+  const void *phi0, *cphi, *vel;
+  void *phi, *kappa;
+  const BCell* cells;
+  Plan p;
+  void* sl[9];
+  void* cv[7];
+  PlanArgs(dcl_batch b, const Plan& plan, const void* phi0_, void* phi_, void* kappa_, const void* vel_)
+      : phi0(phi0_), cphi(phi_), vel(vel_), phi(phi_), kappa(kappa_), cells(b->cells), p(plan) {
+    int n = 0;
+    sl[n++] = &phi0;
+    sl[n++] = &phi;
+    if (!p.kcv) sl[n++] = &kappa;
+    sl[n++] = &vel;
+    sl[n++] = &cells;
+    sl[n++] = &p.tsl;
+    sl[n++] = &p.bsl_bounds;
+    sl[n++] = &p.qsl;
+    sl[n++] = &p.k;
+    void* c[7] = {&cphi, &kappa, &cells, &p.tcv, &p.bcv_bounds, &p.qcv, &p.k};
+    memcpy(cv, c, sizeof(cv));
+  }
+  PlanArgs(const PlanArgs&) = delete;
+};
+
 // enqueue one step with a given configuration
 static int batch_launch(dcl_batch b, int s, int occ, const void* phi0, void* phi, void* kappa, const void* vel,
                         hipStream_t st) {
   Plan p;
   DCL_TRY(make_plan(b, s, occ, p));
-  const BCell* cells = b->cells;
-  void* a1[] = {(void*)&phi0, (void*)&phi, (void*)&vel, (void*)&cells, (void*)&p.tsl, (void*)&p.bsl_bounds,
-                (void*)&p.qsl, (void*)&p.k};
-  DCL_HIP(hipLaunchKernel(p.ksl, p.grid, p.bsl, a1, 0, st));
-  const void* cphi = phi;
-  void* a2[] = {(void*)&cphi, (void*)&kappa, (void*)&cells, (void*)&p.tcv, (void*)&p.bcv_bounds, (void*)&p.qcv,
-                (void*)&p.k};
-  DCL_HIP(hipLaunchKernel(p.kcv, p.grid, p.bcv, a2, 0, st));
+  PlanArgs a(b, p, phi0, phi, kappa, vel);
+  DCL_HIP(hipLaunchKernel(p.ksl, p.grid, p.bsl, a.sl, 0, st));
+  if (p.kcv) DCL_HIP(hipLaunchKernel(p.kcv, p.grid, p.bcv, a.cv, 0, st));
   return 0;
 }
 
@@ -805,12 +815,7 @@ extern "C" int dcl_batch_graph_create(dcl_batch b, const void* phi0, void* phi, 
   if (!graph_exec) return set_error(DCL_ERR_ARG_NULL, "graph_exec is NULL");
   Plan p;
   DCL_TRY(make_plan(b, b->shape, b->occ, p));
-  const BCell* cells = b->cells;
-  const void* cphi = phi;
-  void* a1[] = {(void*)&phi0, (void*)&phi, (void*)&vel, (void*)&cells, (void*)&p.tsl, (void*)&p.bsl_bounds,
-                (void*)&p.qsl, (void*)&p.k};
-  void* a2[] = {(void*)&cphi, (void*)&kappa, (void*)&cells, (void*)&p.tcv, (void*)&p.bcv_bounds, (void*)&p.qcv,
-                (void*)&p.k};
+  PlanArgs a(b, p, phi0, phi, kappa, vel);
   hipGraph_t g;
   DCL_HIP(hipGraphCreate(&g, 0));
   hipKernelNodeParams p1;
@@ -818,15 +823,15 @@ extern "C" int dcl_batch_graph_create(dcl_batch b, const void* phi0, void* phi, 
   p1.func = const_cast<void*>(p.ksl);
   p1.gridDim = p.grid;
   p1.blockDim = p.bsl;
-  p1.kernelParams = a1;
+  p1.kernelParams = a.sl;
   hipKernelNodeParams p2 = p1;
   p2.func = const_cast<void*>(p.kcv);
   p2.blockDim = p.bcv;
-  p2.kernelParams = a2;
+  p2.kernelParams = a.cv;
   hipGraphNode_t n1, n2;
   hipGraphExec_t ex = nullptr;
   hipError_t e = hipGraphAddKernelNode(&n1, g, nullptr, 0, &p1);
-  if (e == hipSuccess) e = hipGraphAddKernelNode(&n2, g, &n1, 1, &p2);
+  if (e == hipSuccess && p.kcv) e = hipGraphAddKernelNode(&n2, g, &n1, 1, &p2);
   if (e == hipSuccess) e = hipGraphInstantiate(&ex, g, nullptr, nullptr, 0);
   (void)hipGraphDestroy(g);
   if (e != hipSuccess) return hip_fail(e, "batch graph build", __FILE__, __LINE__);

@@ -1,6 +1,9 @@
 // step.hip -- one dense level-set update: SL step phi0 -> phi followed by
-// the 19-point (3D) / 9-point (2D) curvature of the new phi.
+// the 19-point (3D) / 9-point (2D) curvature of the new phi.  3D: the SL and
+// the curvature kernel one after the other.  2D with the velocity on phi's
+// window: one fused launch (dcl_step2d.hpp).
 #include "dcl_host.hpp"
+#include "dcl_step2d.hpp"
 
 namespace dcl {
 int sl_launch(const void* phi0, void* phi, const dcl_window* win, const dcl_velocity* vel,
@@ -11,6 +14,65 @@ int check_sl_args(const void* phi0, void* phi, const dcl_window* win, const dcl_
                   int interp, int backtrace);
 int curv_launch(const void* phi, void* kappa, const dcl_window* win, const dcl_icoor* band,
                 int64_t n, void* bv, int precision, int stencil, hipStream_t s);
+int sl_params(const dcl_window* win, const dcl_velocity* vel, double dt, SLP& P);
+
+template <typename T, int INTERP, int BT, int R>
+__global__ __launch_bounds__(Step2<R>::NT) void step2d_k(const T* __restrict__ phi0, T* __restrict__ phi,
+                                                         T* __restrict__ kappa, const T* __restrict__ vel, SLP P,
+                                                         CurvR<T> cr) {
+  __shared__ Step2Lds<T, R> S;
+  step2d_tile<T, INTERP, BT, R>(phi0, phi, kappa, vel, P, cr, (int)blockIdx.x * Step2<R>::OX,
+                                (int)blockIdx.y * Step2<R>::OY, S);
+}
+
+template <int R>
+static dim3 step2d_grid(const KWin& w) {
+  return dim3((w.nx + Step2<R>::OX - 1) / Step2<R>::OX, (w.ny + Step2<R>::OY - 1) / Step2<R>::OY);
+}
+
+// Rows per thread: more rows stage and recompute fewer halo values per node,
+// fewer finish a small window sooner.  The lines lie where they cross, at 2.5
+// and 1.5 blocks per CU (us per FP64 tricubic RK2 step with 1 / 2 / 4 rows,
+// n x n: 128 3.2 / 4.3 / 8.9, 256 4.2 / 4.5 / 6.4, 384 5.7 / 5.6 / 6.6, 512
+// 8.1 / 6.9 / 8.5, 768 15.5 / 13.0 / 11.7, 1024 23.0 / 18.8 / 17.8; FP32 and
+// the trilinear scheme cross at the same sizes).
+template <typename T, int INTERP, int BT>
+static int step2d_launch(const T* phi0, T* phi, T* kappa, const T* vel, const SLP& P, const CurvR<T>& cr,
+                         hipStream_t s) {
+  // at least `halves` half blocks per CU
+  auto fills = [](dim3 g, int halves) { return 2 * (int64_t)g.x * g.y >= (int64_t)halves * device_cus(); };
+  const dim3 block(S2_TX, S2_TY);
+  if (fills(step2d_grid<4>(P.w), 5))
+    hipLaunchKernelGGL((step2d_k<T, INTERP, BT, 4>), step2d_grid<4>(P.w), block, 0, s, phi0, phi, kappa, vel, P, cr);
+  else if (fills(step2d_grid<2>(P.w), 3))
+    hipLaunchKernelGGL((step2d_k<T, INTERP, BT, 2>), step2d_grid<2>(P.w), block, 0, s, phi0, phi, kappa, vel, P, cr);
+  else
+    hipLaunchKernelGGL((step2d_k<T, INTERP, BT, 1>), step2d_grid<1>(P.w), block, 0, s, phi0, phi, kappa, vel, P, cr);
+  DCL_LAUNCHED("step2d");
+  return 0;
+}
+
+template <typename T>
+static int step2d(const void* phi0, void* phi, void* kappa, const dcl_window* win, const dcl_velocity* vel, double dt,
+                  int interp, int backtrace, hipStream_t s) {
+  SLP P;
+  sl_params(win, vel, dt, P);
+  const CurvR<T> cr = curv_recips<T>(win->d.x, win->d.y, 1.0);
+  const T* p0 = static_cast<const T*>(phi0);
+  const T* v = static_cast<const T*>(vel->data);
+  T* p = static_cast<T*>(phi);
+  T* k = static_cast<T*>(kappa);
+  if (interp == DCL_CUBIC && backtrace == DCL_RK2) return step2d_launch<T, DCL_CUBIC, DCL_RK2>(p0, p, k, v, P, cr, s);
+  if (interp == DCL_CUBIC) return step2d_launch<T, DCL_CUBIC, DCL_EULER>(p0, p, k, v, P, cr, s);
+  if (backtrace == DCL_RK2) return step2d_launch<T, DCL_LINEAR, DCL_RK2>(p0, p, k, v, P, cr, s);
+  return step2d_launch<T, DCL_LINEAR, DCL_EULER>(p0, p, k, v, P, cr, s);
+}
+
+// the fused 2D step stages the velocity at phi's nodes; its grid's second
+// dimension holds at most 65535 tiles (two rows each where they are smallest)
+static bool step2d_takes(const dcl_window& w, const dcl_window& v) {
+  return w.n.z < 2 && v.p.x == w.p.x && v.p.y == w.p.y && v.n.x == w.n.x && v.n.y == w.n.y && w.n.y <= 100000;
+}
 }  // namespace dcl
 
 using namespace dcl;
@@ -23,6 +85,9 @@ extern "C" int dcl_levelset_step(const void* phi0, void* phi, void* kappa, const
   if (kappa == phi || kappa == phi0)
     return set_error(DCL_ERR_ARG_WRONG, "kappa must not alias phi or phi0");
   hipStream_t s = as_stream(stream);
+  if (step2d_takes(*win, vel->win))
+    return precision == DCL_F64 ? step2d<double>(phi0, phi, kappa, win, vel, dt, interp, backtrace, s)
+                                : step2d<float>(phi0, phi, kappa, win, vel, dt, interp, backtrace, s);
   DCL_TRY(sl_launch(phi0, phi, win, vel, nullptr, 0, nullptr, dt, precision, interp, backtrace, s));
   return curv_launch(phi, kappa, win, nullptr, 0, nullptr, precision, DCL_CURV_STD, s);
 }

@@ -386,7 +386,8 @@ int dcl_error_norms(const void *a, int prec_a, const void *b, int prec_b, int64_
  * the cells' windows are packed back to back in one phi buffer, one kappa
  * buffer and one velocity buffer (dim components per node, as a velgrid),
  * cut into tiles, and one step is two persistent launches over the packed
- * tile list (SL then curvature, as dcl_levelset_step per cell), each XCD
+ * tile list (SL then curvature, as dcl_levelset_step per cell; in 2D one
+ * launch does both), each XCD
  * working through a chunk of the list of about equal cost, so cells of
  * uneven sizes load the whole chip.  A batch holds 3D cells or 2D cells, not
  * both.  No counterpart in the reference.  The velocity of each cell shares
@@ -412,7 +413,7 @@ int dcl_batch_set_dt(dcl_batch batch, const double *dt);
  * shape (tile[] of dcl_batch_get_config), shape 6..11 = the curvature tiles
  * of shape - 6 with the SL step over 32 x 8 columns of the cell class's
  * z-chunk staged in an LDS ring; occupancy 0..2 -> 2, 4, 8 resident blocks
- * per CU.  2D batches use 64 x 4 node tiles whatever the shape. */
+ * per CU.  2D batches use one tile whatever the shape. */
 int dcl_batch_set_config(dcl_batch batch, int shape, int occupancy);
 int dcl_batch_get_config(dcl_batch batch, int *shape, int *occupancy, int32_t tile[3],
                          int *blocks);
@@ -451,7 +452,7 @@ int dcl_batch_autotune(dcl_batch batch, const void *phi0, void *phi, void *kappa
                        const void *vel, int reps, double *ms_table, double *zc_table,
                        double *claim_table, double *best_ms, void *stream);
 /* One step with these buffers recorded as an instantiated hipGraph (two
- * kernel nodes); launch it with dcl_batch_graph_launch. */
+ * kernel nodes, in 2D one); launch it with dcl_batch_graph_launch. */
 int dcl_batch_graph_create(dcl_batch batch, const void *phi0, void *phi, void *kappa,
                            const void *vel, void **graph_exec);
 int dcl_batch_graph_launch(void *graph_exec, void *stream);

@@ -292,6 +292,48 @@ def test_levelset_step_planes_equal_per_node(dev, dtype, dim):
         assert torch.equal(a, b) and torch.equal(ka, kb)
 
 
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+@pytest.mark.parametrize("interp,bt", [("cubic", "rk2"), ("linear", "euler"), ("linear", "rk2")])
+@pytest.mark.parametrize("n,layout", [((5, 5), 2), ((62, 14), 2), ((63, 15), 1), ((61, 17), 3), ((125, 6), 2),
+                                      ((7, 300), 1), ((500, 430), 2), ((833, 801), 3)])
+def test_levelset_step_2d_tiles(dev, dtype, interp, bt, n, layout):
+    """The fused 2D step around its tile edges, at each number of rows per
+    thread, with every velocity layout (planes, (u, v), (p, u, v)) and
+    departures on both sides of the staged halo: phi against the oracle, kappa
+    against the curvature kernel on the same phi within the rounding of the
+    terms of its sum (33 unit roundoffs per evaluation)."""
+    rng = np.random.default_rng(n[0] + n[1])
+    h = 1.0 / (max(n) - 1)
+    win = D.GridWindow((3, -2, 0), (n[0], n[1], 1), (h, 1.2 * h, h))
+    y, x = np.meshgrid(np.arange(float(n[1])), np.arange(float(n[0])), indexing="ij")
+    phi0 = np.hypot(x - 0.4 * n[0], y - 0.55 * n[1]) - 0.3 * min(n) + 0.2 * np.sin(0.3 * x + 0.2 * y)
+    vel = rng.normal(size=2) + np.stack([np.sin(0.11 * y + 0.05 * x), np.cos(0.07 * x - 0.1 * y)], axis=-1)
+    phi0, vel = rounded(phi0, dtype), rounded(vel, dtype)
+    dt = 2.6 * h / np.abs(vel).max()
+    if layout == 1:
+        dvel, kw = to_dev(np.moveaxis(vel, -1, 0), dtype), dict(planes=True)
+    elif layout == 2:
+        dvel, kw = to_dev(vel, dtype), {}
+    else:
+        dvel, kw = to_dev(np.concatenate([np.full(vel.shape[:2] + (1,), np.nan), vel], axis=-1), dtype), dict(udof=1)
+    phi, kap = D.levelset_step(to_dev(phi0, dtype), dvel, win, dt, interp, bt, **kw)
+    ref = O.sl_advect(phi0, vel, owin(win), dt, IM[interp], BM[bt])
+    assert rel_max(to_np(phi), ref) <= TOL[dtype]
+    other = to_np(D.curvature(phi, win))
+    p = to_np(phi)
+    px, py = (p[1:-1, 2:] - p[1:-1, :-2]) / (2 * win.d[0]), (p[2:, 1:-1] - p[:-2, 1:-1]) / (2 * win.d[1])
+    pxx = (p[1:-1, 2:] - 2 * p[1:-1, 1:-1] + p[1:-1, :-2]) / win.d[0] ** 2
+    pyy = (p[2:, 1:-1] - 2 * p[1:-1, 1:-1] + p[:-2, 1:-1]) / win.d[1] ** 2
+    pxy = (p[2:, 2:] + p[:-2, :-2] - p[2:, :-2] - p[:-2, 2:]) / (4 * win.d[0] * win.d[1])
+    # the sums of p are rounded in the kernels' precision, the same in both
+    mag = (np.abs(pxx) * py ** 2 + 2 * np.abs(px * py * pxy) + np.abs(pyy) * px ** 2) / (px ** 2 + py ** 2) ** 1.5
+    lost = 4 * np.abs(p).max() * (1 / win.d[0] ** 2 + 1 / win.d[1] ** 2) / np.sqrt(px ** 2 + py ** 2)
+    u = 2.0 ** (-53 if dtype == torch.float64 else -24)
+    diff = np.abs(to_np(kap) - other)
+    assert diff[0].max() == diff[-1].max() == diff[:, 0].max() == diff[:, -1].max() == 0
+    assert np.all(diff[1:-1, 1:-1] <= 66 * u * (mag + u * lost))
+
+
 def test_zalesak_c1_revolution_fp64(dev):
     """C1 (128^2 Zalesak disk, rigid rotation, dt = 1/628) for 157 steps (a
     quarter revolution) in reference mode (Euler + Bilinear2D) and config mode
