@@ -164,17 +164,22 @@ __global__ __launch_bounds__(shape_of(S).tx * shape_of(S).ty) void batch_sl_k(
 // ring columns of the batch: 32 x 8 nodes, the cell's z-chunk, velocity staged in FP32
 constexpr int RING_TX = 32, RING_TY = 8;
 
+template <typename T>
+constexpr int batch_vel() {
+  return sizeof(T) == 4 ? RV_STAGED : RV_GATHER;
+}
+
 template <typename T, int INTERP, int BT>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ring_waves<T, sizeof(T) == 4>(), 8))) void
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(ring_waves<T, batch_vel<T>()>(), 8))) void
 batch_ring_k(const T* __restrict__ phi0, T* __restrict__ phi,
                                                       const T* __restrict__ vel, const BCell* __restrict__ cells,
                                                       const int4* __restrict__ tiles,
                                                       const int* __restrict__ bounds, WorkQ* __restrict__ q, int k) {
   typedef typename RingFor<T, RING_TX, RING_TY>::type G;
   typedef VelGeom<RING_TX, RING_TY, G::VRP, G::VPP> V;
-  constexpr bool VL = sizeof(T) == 4;
+  constexpr int VM = batch_vel<T>();
   __shared__ T ring[RG_R * G::PP];
-  __shared__ T vr[VL ? VR_R * 3 * V::PP : 1];
+  __shared__ T vr[VM == RV_STAGED ? VR_R * 3 * V::PP : 1];
   claim_tiles(q, bounds, k, [&](int t) {
     const int4 tl = tiles[t];
     const BCell c = cells[tl.x];
@@ -182,7 +187,7 @@ batch_ring_k(const T* __restrict__ phi0, T* __restrict__ phi,
     const unsigned nodes = (unsigned)c.nx * c.ny * c.nz;
     const rsrc_t rp = make_rsrc(phi0 + c.phi_off, nodes * (unsigned)sizeof(T));
     const rsrc_t rv = make_rsrc(vel + c.vel_off, 3u * nodes * (unsigned)sizeof(T));
-    ring_column<T, INTERP, BT, G, VL>(phi0 + c.phi_off, phi + c.phi_off, rp, rv, P, tl.y, tl.z, tl.w, c.zc, ring,
+    ring_column<T, INTERP, BT, G, VM>(phi0 + c.phi_off, phi + c.phi_off, rp, rv, P, tl.y, tl.z, tl.w, c.zc, ring,
                                       vr);
   });
 }

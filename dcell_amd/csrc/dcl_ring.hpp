@@ -272,6 +272,11 @@ __device__ __forceinline__ void sl_dep3_ring(rsrc_t rv, const T* vr, const int s
   for (int a = 0; a < 3; ++a) S[a] = Xd[a] - (double)V2[a] * P.c[a];
 }
 
+// where a ring kernel's velocity comes from: gathered per node (any layout
+// with the components stored per node), staged in the velocity ring, or
+// component planes (dof 1), gathered with the previous plane's corners carried
+enum RingVel { RV_GATHER = 0, RV_STAGED = 1, RV_PLANES = 2 };
+
 // a phi value of the column's output: FP64 nontemporally (the 256^3 step
 // with the curvature after it measured 1% faster, the FP32 kernels as much
 // slower)
@@ -288,11 +293,12 @@ __device__ __forceinline__ void ring_put(T* p, T v) {
 // Every thread of the block calls it (it holds barriers) and it ends on a
 // barrier, so a block may run it for one column after another with the same
 // ring (RG_R * G::PP values).
-template <typename T, int INTERP, int BT, typename G, bool VL>
+template <typename T, int INTERP, int BT, typename G, int VM>
 __device__ __forceinline__ void ring_column(const T* __restrict__ phi0, T* __restrict__ phi, rsrc_t rp,
                                             rsrc_t rv, const SLP& P, int x0, int y0, int z0, int zc, T* ring,
                                             T* vr) {
   typedef VelGeom<G::TX, G::TY, G::VRP, G::VPP> V;
+  constexpr bool VL = VM == RV_STAGED, planes = VM == RV_PLANES;
   const int nx = P.w.nx, ny = P.w.ny, nz = P.w.nz;
   const int z1 = min(nz, z0 + zc);
   const int tid = threadIdx.x + G::TX * threadIdx.y;
@@ -324,8 +330,14 @@ __device__ __forceinline__ void ring_column(const T* __restrict__ phi0, T* __res
   // node faces are loaded while this plane is worked (nf), so a plane waits
   // on one round trip to memory (the RK2 midpoint's corners) instead of
   // two: 0.327 -> 0.320 ms at 256^3 (in FP32 it was slower)
-  const bool planes = P.v.dof == 1;
   T wc = T(0);
+  MacCarry<T> mc;
+#pragma unroll
+  for (int c = 0; c < 3; ++c) {
+    mc.vo[c] = -1;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) mc.hi[c][q] = T(0);
+  }
   NodeFaces<T> nf = {T(0), T(0), T(0), T(0), T(0)};
   for (int k = z0; k < z1; ++k) {
     const int zn = k + RG_H + 1;
@@ -341,11 +353,11 @@ __device__ __forceinline__ void ring_column(const T* __restrict__ phi0, T* __res
         ring_put<T>(phi + id, phi0[id]);
       } else {
         double S[3];
-        if (VL) {
+        if constexpr (VL) {
           const int b = (k - z0) % VR_R;
           const int sl[4] = {b, (b + 1) % VR_R, (b + 2) % VR_R, (b + 3) % VR_R};
           sl_dep3_ring<T, BT, V>(rv, vr, sl, P, i, j, k, x0, y0, S);
-        } else if (planes) {
+        } else if constexpr (planes) {
           const int vz0 = P.v.w.pz, vz1 = P.v.w.pz + P.v.w.nz - 2;
           const bool pf = k - 1 >= max(z0, 2);  // the previous plane was computed here
           const bool carry = pf && clampi(P.w.pz + k, vz0, vz1) == clampi(P.w.pz + k - 1, vz0, vz1) + 1;
@@ -369,7 +381,14 @@ __device__ __forceinline__ void ring_column(const T* __restrict__ phi0, T* __res
           } else {
             node_vel_planes_z<T>(rv, P.v, X, Y, Z, carry, wc, V);
           }
-          sl_dep3_from<T, BT>(rv, P, X, Y, Z, V, S);
+          const double Xd[3] = {(double)X, (double)Y, (double)Z};
+          if constexpr (BT == DCL_RK2) {
+            const double Xm[3] = {Xd[0] - (double)V[0] * P.ch[0], Xd[1] - (double)V[1] * P.ch[1],
+                                  Xd[2] - (double)V[2] * P.ch[2]};
+            mac_vel_planes_z<T>(rv, P.v, Xm, mc, V);
+          }
+#pragma unroll
+          for (int a = 0; a < 3; ++a) S[a] = Xd[a] - (double)V[a] * P.c[a];
           if constexpr (sizeof(T) == 8) {
             if (k + 1 < z1 && k + 1 <= nz - 3) nf = node_faces_planes<T>(rv, P.v, X, Y, Z + 1);
           }
@@ -389,22 +408,23 @@ __device__ __forceinline__ void ring_column(const T* __restrict__ phi0, T* __res
 // kernel's LDS (40 KB per 256-thread block) admits 4 blocks per CU, and
 // asking for 4 waves per SIMD brings its registers from 136 to 104 (no
 // spills), 7% faster at 384^3; the others keep the compiler's choice.
-template <typename T, bool VL>
+template <typename T, int VM>
 constexpr int ring_waves() {
-  return sizeof(T) == 4 && VL ? 4 : 1;
+  return sizeof(T) == 4 && VM == RV_STAGED ? 4 : 1;
 }
 
 // grid: tiles_x * tiles_y * nzc blocks of TX x TY threads (XCD-remapped so
-// each XCD walks neighbouring columns), each walking zch planes.  VL:
-// velocity staged too (velocity window = phi window, 3 components, udof 0).
-template <typename T, int INTERP, int BT, int TX, int TY, bool VL>
-__global__ __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(ring_waves<T, VL>(), 8))) void sl_ring3d(
+// each XCD walks neighbouring columns), each walking zch planes.  VM:
+// RV_STAGED needs velocity window = phi window, 3 components, udof 0;
+// RV_PLANES takes dof 1, RV_GATHER the others.
+template <typename T, int INTERP, int BT, int TX, int TY, int VM>
+__global__ __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(ring_waves<T, VM>(), 8))) void sl_ring3d(
     const T* __restrict__ phi0, T* __restrict__ phi, const T* __restrict__ vel, SLP P, unsigned tiles_x,
     unsigned tiles_y, unsigned nzc, int zch, unsigned pbytes, unsigned vbytes) {
   typedef typename RingFor<T, TX, TY>::type G;
   typedef VelGeom<TX, TY, G::VRP, G::VPP> V;
   __shared__ T ring[RG_R * G::PP];
-  __shared__ T vr[VL ? VR_R * 3 * V::PP : 1];
+  __shared__ T vr[VM == RV_STAGED ? VR_R * 3 * V::PP : 1];
   const unsigned nb = tiles_x * tiles_y * nzc;
   unsigned lb = blockIdx.x;
   {
@@ -412,7 +432,7 @@ __global__ __launch_bounds__(TX * TY) __attribute__((amdgpu_waves_per_eu(ring_wa
     if (per != 0 && lb < per * 8u) lb = (lb % 8u) * per + lb / 8u;
   }
   const unsigned tx = lb % tiles_x, ty = (lb / tiles_x) % tiles_y, zc = lb / (tiles_x * tiles_y);
-  ring_column<T, INTERP, BT, G, VL>(phi0, phi, make_rsrc(phi0, pbytes), make_rsrc(vel, vbytes), P, (int)tx * TX,
+  ring_column<T, INTERP, BT, G, VM>(phi0, phi, make_rsrc(phi0, pbytes), make_rsrc(vel, vbytes), P, (int)tx * TX,
                                     (int)ty * TY, (int)zc * zch, zch, ring, vr);
 }
 

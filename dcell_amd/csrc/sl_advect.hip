@@ -111,8 +111,9 @@ static int launch_sl_b(const void* phi0, void* phi, const void* vel, const SLP& 
     const bool same = P.v.w.px == P.w.px && P.v.w.py == P.w.py && P.v.w.pz == P.w.pz && P.v.w.nx == P.w.nx &&
                       P.v.w.ny == P.w.ny && P.v.w.nz == P.w.nz && P.v.dof == 3 && P.v.udof == 0;
     const bool vl = same && (ve ? atoi(ve) != 0 : (sizeof(T) == 4 || INTERP == DCL_LINEAR));
+    const int vm = P.v.dof == 1 ? RV_PLANES : vl ? RV_STAGED : RV_GATHER;
 #define DCL_RING(GI, TXV, TYV, VLV)                                                                      \
-  if (g == GI && vl == VLV) {                                                                            \
+  if (g == GI && vm == VLV) {                                                                            \
     const unsigned tx = (P.w.nx + TXV - 1) / TXV, ty = (P.w.ny + TYV - 1) / TYV;                         \
     int zc = 32;                                                                                         \
     while (zc > 8 && (int64_t)tx * ty * ((P.w.nz + zc - 1) / zc) < 4 * (int64_t)device_cus()) zc /= 2;   \
@@ -120,12 +121,12 @@ static int launch_sl_b(const void* phi0, void* phi, const void* vel, const SLP& 
     hipLaunchKernelGGL((sl_ring3d<T, INTERP, BT, TXV, TYV, VLV>), dim3(tx * ty * nzc), dim3(TXV, TYV), 0, \
                        s, p0, static_cast<T*>(phi), v, P, tx, ty, nzc, zc, pb, vb);                      \
   }
-    DCL_RING(0, 16, 16, false)
-    DCL_RING(1, 32, 8, false)
-    DCL_RING(2, 64, 4, false)
-    DCL_RING(0, 16, 16, true)
-    DCL_RING(1, 32, 8, true)
-    DCL_RING(2, 64, 4, true)
+#define DCL_RING3(GI, TXV, TYV) \
+  DCL_RING(GI, TXV, TYV, RV_GATHER) DCL_RING(GI, TXV, TYV, RV_STAGED) DCL_RING(GI, TXV, TYV, RV_PLANES)
+    DCL_RING3(0, 16, 16)
+    DCL_RING3(1, 32, 8)
+    DCL_RING3(2, 64, 4)
+#undef DCL_RING3
 #undef DCL_RING
     DCL_LAUNCHED("sl_ring3d");
     return 0;
