@@ -474,10 +474,12 @@ __global__ __launch_bounds__(256) void adj_prepare_k(const T* __restrict__ vel, 
 // LDS box of lam (the column plus the reach WR) that no other wave touches.
 // So the scatter is a plain LDS read-add-write per lane: a float atomic in
 // LDS costs about 3 cycles per active lane (a 64-lane ds_add_f32 takes ~190
-// cycles of a CU's LDS, a ds_write 5), and that was this step's cost.  Two
-// lanes of one instruction may write the same word only when their stencil
-// corners coincide (departures that converge); such lanes are found per
-// plane with a tag table and take LDS atomics instead.  x-neighbour lanes
+// cycles of a CU's LDS, a ds_write 5), and that was this step's cost.  The
+// four stencil planes of one (x, y) entry are read, added to and written
+// together, so a node's 64 words cost 16 waits for LDS instead of 64; two
+// lanes of one such group may write the same word only when their stencils'
+// (x, y) corners coincide (departures that converge); such lanes are found
+// per plane with a tag table and take LDS atomics instead.  x-neighbour lanes
 // whose corners are 1..3 words apart combine their shared words with DPP row
 // shifts before writing (as in sl_adjoint_k).  Stencils that leave the box
 // (departures of 2 cells or more) add into lam with HBM atomics.  The box and
@@ -492,7 +494,7 @@ __global__ __launch_bounds__(64) void adj_step_k(const T* __restrict__ phi0, con
   constexpr int OFF = INTERP == DCL_CUBIC ? -1 : 0;
   const Frac4<T, INTERP>* __restrict__ rf = static_cast<const Frac4<T, INTERP>*>(rfv);
   __shared__ T box_s[WBOX];
-  __shared__ int tag_s[NTAG];
+  __shared__ int tag_s[WBX * WBY + 1];
   typedef __attribute__((address_space(3))) T lds_T;
   typedef __attribute__((address_space(3))) int lds_int;
   volatile lds_T* box = (volatile lds_T*)box_s;
@@ -569,9 +571,9 @@ __global__ __launch_bounds__(64) void adj_step_k(const T* __restrict__ phi0, con
     const bool in_box =
         act && bx0 >= 0 && bx0 + NP <= WBX && by0 >= 0 && by0 + NP <= WBY && bz0 >= 0 && bz0 + NP <= WBZ;
     const int key = in_box ? (bz0 * WBY + by0) * WBX + bx0 + 1 : 0;
-    // lanes sharing a stencil corner: each tags its slot, lanes that lose
-    // mark the slot, and every lane whose slot ends marked takes atomics
-    const int slot = key & (NTAG - 1);
+    // lanes sharing an (x, y) corner: each tags its slot, lanes that lose mark
+    // the slot, and every lane whose slot ends marked takes atomics
+    const int slot = in_box ? by0 * WBX + bx0 : 0;
     if (in_box) tag[slot] = lane;
     const bool lost = in_box && tag[slot] != lane;
     if (lost) tag[slot] = -1;
@@ -587,58 +589,88 @@ __global__ __launch_bounds__(64) void adj_step_k(const T* __restrict__ phi0, con
     T G[3] = {T(0), T(0), T(0)};
     // the stencil rows with buffer loads (a row of 4 values is one 16-byte
     // load in FP32, two in FP64; inactive lanes read the window's first row),
-    // all stencil planes in flight at once in FP32, one at a time in FP64
+    // all of them in flight at once in FP32, the planes of one y at a time in
+    // FP64
     const int vo = act ? ((b[2] + OFF) * Z + (b[1] + OFF) * Y + (b[0] + OFF)) * (int)sizeof(T) : 0;
-    constexpr int KP = sizeof(T) == 4 ? NP : 1;
-#pragma unroll 1
-    for (int k0 = 0; k0 < NP; k0 += KP) {
-      T rows[KP][4][4];
+    auto load_rows = [&](int jj, T (&rows)[NP][4]) {
 #pragma unroll
-      for (int dk = 0; dk < KP; ++dk)
+      for (int kk = 0; kk < NP; ++kk) {
+        const int so = (kk * Z + jj * Y) * (int)sizeof(T);
+        if (NP == 4) BL<T>::four(rp, vo, so, rows[kk]);
+        else BL<T>::two(rp, vo, so, rows[kk]);
+      }
+    };
+    // the rows of y entry jj (weights wy, dwy): the gradient's sums, and the
+    // scatter of the row's words
+    auto work_rows = [&](int jj, T wy, T dwy, const T (&rows)[NP][4]) {
+      T add[NP][4], word0[NP];
 #pragma unroll
-        for (int jj = 0; jj < NP; ++jj) {
-          const int so = ((k0 + dk) * Z + jj * Y) * (int)sizeof(T);
-          if (NP == 4) BL<T>::four(rp, vo, so, rows[dk][jj]);
-          else BL<T>::two(rp, vo, so, rows[dk][jj]);
+      for (int kk = 0; kk < NP; ++kk) {
+        const T wyz = wy * w[2][kk];
+#pragma unroll
+        for (int ii = 0; ii < NP; ++ii) add[kk][ii] = g * w[0][ii] * wyz;
+        word0[kk] = add[kk][0];
+#pragma unroll
+        for (int d = 1; d < NP; ++d) {
+          const T o = lane_from_lower(add[kk][d], d);
+          if (lo_m[d]) word0[kk] += o;
         }
-#pragma unroll
-      for (int dk = 0; dk < KP; ++dk)
-#pragma unroll
-        for (int jj = 0; jj < NP; ++jj) {
-          const int kk = k0 + dk;
-          const T wyz = w[1][jj] * w[2][kk];
-          T add[4];
-#pragma unroll
-          for (int ii = 0; ii < NP; ++ii) add[ii] = g * w[0][ii] * wyz;
-          T word0 = add[0];
-#pragma unroll
-          for (int d = 1; d < NP; ++d) {
-            const T o = lane_from_lower(add[d], d);
-            if (lo_m[d]) word0 += o;
-          }
-          if (act) {
-            T rx = T(0), rd = T(0);
-#pragma unroll
-            for (int ii = 0; ii < NP; ++ii) {
-              const T f = rows[dk][jj][ii];
-              rx += w[0][ii] * f;
-              rd += dw[0][ii] * f;
-            }
-            G[0] += rd * wyz;
-            G[1] += rx * dw[1][jj] * w[2][kk];
-            G[2] += rx * w[1][jj] * dw[2][kk];
-          }
-          const int wo = ((bz0 + kk) * WBY + (by0 + jj)) * WBX + bx0;
+        if (act) {
+          T rx = T(0), rd = T(0);
 #pragma unroll
           for (int ii = 0; ii < NP; ++ii) {
-            const T v = ii == 0 ? word0 : add[ii];
-            const bool mine = ii == 0 || !up_m[ii];
-            if (plain && mine) box[wo + ii] = box[wo + ii] + v;
-            if (shared && mine) atomicAdd(&box_s[wo + ii], v);
-            if (act && !in_box)
-              atomic_add(&lam[(b[2] + OFF + kk) * Z + (b[1] + OFF + jj) * Y + (b[0] + OFF + ii)], add[ii]);
+            const T f = rows[kk][ii];
+            rx += w[0][ii] * f;
+            rd += dw[0][ii] * f;
           }
+          G[0] += rd * wyz;
+          G[1] += rx * dwy * w[2][kk];
+          G[2] += rx * wy * dw[2][kk];
         }
+      }
+      const int wo = (bz0 * WBY + (by0 + jj)) * WBX + bx0;
+#pragma unroll
+      for (int ii = 0; ii < NP; ++ii) {
+        const bool mine = ii == 0 || !up_m[ii];
+        if (plain && mine) {
+          T old[NP];
+#pragma unroll
+          for (int kk = 0; kk < NP; ++kk) old[kk] = box[wo + kk * WBX * WBY + ii];
+#pragma unroll
+          for (int kk = 0; kk < NP; ++kk)
+            box[wo + kk * WBX * WBY + ii] = old[kk] + (ii == 0 ? word0[kk] : add[kk][ii]);
+        }
+        if (shared && mine) {
+#pragma unroll
+          for (int kk = 0; kk < NP; ++kk)
+            atomicAdd(&box_s[wo + kk * WBX * WBY + ii], ii == 0 ? word0[kk] : add[kk][ii]);
+        }
+        if (act && !in_box) {
+#pragma unroll
+          for (int kk = 0; kk < NP; ++kk)
+            atomic_add(&lam[(b[2] + OFF + kk) * Z + (b[1] + OFF + jj) * Y + (b[0] + OFF + ii)], add[kk][ii]);
+        }
+      }
+    };
+    if constexpr (sizeof(T) == 4) {
+      T rows[NP][NP][4];
+#pragma unroll
+      for (int jj = 0; jj < NP; ++jj) load_rows(jj, rows[jj]);
+#pragma unroll
+      for (int jj = 0; jj < NP; ++jj) work_rows(jj, w[1][jj], dw[1][jj], rows[jj]);
+    } else {
+#pragma unroll 1
+      for (int jj = 0; jj < NP; ++jj) {
+        T rows[NP][4];
+        load_rows(jj, rows);
+        T wy = w[1][0], dwy = dw[1][0];
+#pragma unroll
+        for (int m = 1; m < NP; ++m) {
+          wy = jj == m ? w[1][m] : wy;
+          dwy = jj == m ? dw[1][m] : dwy;
+        }
+        work_rows(jj, wy, dwy, rows);
+      }
     }
     if (act) {
 #pragma unroll
