@@ -44,6 +44,7 @@ struct MacState {
   T V[3];
   T dV[3][3];   // dV[c][axis]
   int base[3];  // element offset of corner (0,0,0) of component c (includes c + udof)
+  int bi[3][3]; // its node [c][axis], window-local
   T f[3][3];    // fractions [c][axis]
 };
 
@@ -69,14 +70,25 @@ __device__ __forceinline__ void mac_state(const T* __restrict__ vel, const KVel&
       const double sh = a == c ? 0.5 : 0.0;
       const double fl = floor(X[a] + sh);
       bi[a] = (int)fl - lo[a];
+      m.bi[c][a] = bi[a];
       fr[a] = (T)(X[a] - fl + sh);
       m.f[c][a] = fr[a];
     }
     const int base = bi[2] * sz + bi[1] * sy + bi[0] * sx + v.udof + c;
     m.base[c] = base;
     const T* b = vel + base;
-    const T f000 = b[0], f100 = b[sx], f010 = b[sy], f110 = b[sy + sx];
-    const T f001 = b[sz], f101 = b[sz + sx], f011 = b[sz + sy], f111 = b[sz + sy + sx];
+    T f000, f100, f010, f110, f001, f101, f011, f111;
+    if (sizeof(T) == 4 && v.dof == 3) {
+      // an x pair is the first and last of four neighbouring values, one load
+      typedef T quad __attribute__((ext_vector_type(4), aligned(sizeof(T))));
+      const quad q0 = *reinterpret_cast<const quad*>(b), q1 = *reinterpret_cast<const quad*>(b + sy);
+      const quad q2 = *reinterpret_cast<const quad*>(b + sz), q3 = *reinterpret_cast<const quad*>(b + sz + sy);
+      f000 = q0.x, f100 = q0.w, f010 = q1.x, f110 = q1.w;
+      f001 = q2.x, f101 = q2.w, f011 = q3.x, f111 = q3.w;
+    } else {
+      f000 = b[0], f100 = b[sx], f010 = b[sy], f110 = b[sy + sx];
+      f001 = b[sz], f101 = b[sz + sx], f011 = b[sz + sy], f111 = b[sz + sy + sx];
+    }
     const T x1 = fr[0], x0 = T(1) - fr[0], y1 = fr[1], y0 = T(1) - fr[1], z1 = fr[2], z0 = T(1) - fr[2];
     // values along x for the four (y, z) rows
     const T r00 = x0 * f000 + x1 * f100, r10 = x0 * f010 + x1 * f110;
@@ -164,9 +176,8 @@ __device__ __forceinline__ void mac_scatter_lanes(T* __restrict__ gvel, const KV
 }
 
 // A wave's lanes are a 16 x 4 plane of nodes (its 16-lane DPP rows are x
-// rows, lanes ABX apart are y neighbours); adj_finish_k's blocks stack ABZ
-// such planes.
-constexpr int ABX = 16, ABY = 4, ABZ = 4;
+// rows, lanes ABX apart are y neighbours).
+constexpr int ABX = 16, ABY = 4;
 static_assert(ABX * ABY == 64, "a wave is one z plane of the block: lanes ABX apart are y neighbours");
 
 // One wave per block: its 16 x 4 lanes own a 16 x 4 column of nodes and walk
@@ -470,7 +481,7 @@ __global__ __launch_bounds__(256) void adj_prepare_k(const T* __restrict__ vel, 
 }
 
 // One adjoint step from the record.  A block is one wave: its 16 x 4 lanes
-// own a 16 x 4 column of nodes and walk AWZ planes of it, scattering into an
+// own a 16 x 4 column of nodes and walk PZ planes of it, scattering into an
 // LDS box of lam (the column plus the reach WR) that no other wave touches.
 // So the scatter is a plain LDS read-add-write per lane: a float atomic in
 // LDS costs about 3 cycles per active lane (a 64-lane ds_add_f32 takes ~190
@@ -485,12 +496,22 @@ __global__ __launch_bounds__(256) void adj_prepare_k(const T* __restrict__ vel, 
 // (departures of 2 cells or more) add into lam with HBM atomics.  The box and
 // tag accesses are volatile: the lanes read words other lanes wrote, which
 // the compiler must not forward from a lane's own earlier store.
-template <typename T, int INTERP>
+//
+// lam_next is zero away from the interface in the first steps back from a
+// loss that lives there, so it is read two planes ahead and the rest only
+// where it is not zero: a plane without such a lane ends there, and a column
+// without one touches no record, sum or box. 128^3 FP32, per step:
+// 87 us with every load and wait, 60 with the planes added together, 50 with
+// the skips for a gradient within 6 cells of a sphere's surface and 117
+// (before: 160) for one that is nonzero everywhere, where the box's flush
+// (3.6 atomics per node) and the LDS round trips are about a third each.
+template <typename T, int INTERP, int PZ>
 __global__ __launch_bounds__(64) void adj_step_k(const T* __restrict__ phi0, const int4* __restrict__ rb,
                                                  const void* __restrict__ rfv,
                                                  const T* __restrict__ lam_next, T* __restrict__ lam,
                                                  T* __restrict__ hsum, AdjP P) {
   constexpr int NP = INTERP == DCL_CUBIC ? 4 : 2;
+  constexpr int WBZ = PZ + 2 * WR, WBOX = WBX * WBY * WBZ;
   constexpr int OFF = INTERP == DCL_CUBIC ? -1 : 0;
   const Frac4<T, INTERP>* __restrict__ rf = static_cast<const Frac4<T, INTERP>*>(rfv);
   __shared__ T box_s[WBOX];
@@ -500,29 +521,27 @@ __global__ __launch_bounds__(64) void adj_step_k(const T* __restrict__ phi0, con
   volatile lds_T* box = (volatile lds_T*)box_s;
   volatile lds_int* tag = (volatile lds_int*)tag_s;
   const int lane = threadIdx.x;
-  for (int t = lane; t < WBOX; t += 64) box[t] = T(0);
+  bool boxed = false;  // the box is in use (uniform)
 
-  const int ox = blockIdx.x * ABX, oy = blockIdx.y * ABY, oz = blockIdx.z * AWZ;
+  const int ox = blockIdx.x * ABX, oy = blockIdx.y * ABY, oz = blockIdx.z * PZ;
   const int i = ox + (lane & (ABX - 1)), j = oy + lane / ABX;
   const int nx = P.w.nx, ny = P.w.ny, nz = P.w.nz;
   const int Y = nx, Z = nx * ny;
   const rsrc_t rp = make_rsrc(phi0, (unsigned)((int64_t)nx * ny * nz * (int64_t)sizeof(T)));
-  // a node's record, lam_next and sensitivity sum so far, loaded together,
-  // the next plane's while this plane's stencils are worked
+  // lam_next two planes ahead; an active node's record and sensitivity sum so
+  // far one plane ahead, while this plane's stencils are worked
   auto inner_at = [&](int k) {
     return i >= 2 && i <= nx - 3 && j >= 2 && j <= ny - 3 && k >= 2 && k <= nz - 3;
   };
-  T ng = T(0), nh[3] = {T(0), T(0), T(0)};
+  auto load_lam = [&](int k) {
+    return i < nx && j < ny && k < nz && k < oz + PZ ? lam_next[k * Z + j * Y + i] : T(0);
+  };
+  T nh[3] = {T(0), T(0), T(0)};
   int4 nq = make_int4(0, 0, 0, 0);
   Frac4<T, INTERP> nf = {0, 0, 0, 0};
-  auto load_node = [&](int k) {
-    ng = T(0);
-    nh[0] = nh[1] = nh[2] = T(0);
-    nq = make_int4(0, 0, 0, 0);
-    nf = Frac4<T, INTERP>{0, 0, 0, 0};
-    if (inner_at(k)) {
+  auto load_node = [&](int k, T g) {
+    if (g != T(0) && inner_at(k)) {
       const int id = k * Z + j * Y + i;
-      ng = lam_next[id];
       nq = rb[id];
       nf = rf[id];
       const T* hs = hsum + 3 * (int64_t)id;
@@ -530,23 +549,27 @@ __global__ __launch_bounds__(64) void adj_step_k(const T* __restrict__ phi0, con
       for (int a = 0; a < 3; ++a) nh[a] = hs[a];
     }
   };
-  load_node(oz);
+  T ng = load_lam(oz), nng = load_lam(oz + 1);
+  load_node(oz, ng);
 #pragma unroll 1
-  for (int kz = 0; kz < AWZ; ++kz) {
+  for (int kz = 0; kz < PZ; ++kz) {
     const int k = oz + kz;
-    const bool valid = i < nx && j < ny && k < nz;
-    const bool inner = valid && inner_at(k);
+    const bool inner = inner_at(k);  // lanes past the window carry lam_next 0
     const int id = k * Z + j * Y + i;
-    if (valid && !inner) {
-      const T gb = lam_next[id];
-      if (gb != T(0)) atomic_add(&lam[id], gb);
-    }
     const T g = ng, h0[3] = {nh[0], nh[1], nh[2]};
     const int4 q = nq;
     const Frac4<T, INTERP> f4 = nf;
-    if (kz + 1 < AWZ) load_node(k + 1);
+    ng = nng;
+    if (kz + 1 < PZ) load_node(k + 1, ng);
+    nng = load_lam(k + 2);
+    if (!inner && g != T(0)) atomic_add(&lam[id], g);
     T* hs = hsum + 3 * (int64_t)id;
     const bool act = inner && g != T(0);
+    if (__ballot(act) == 0ull) continue;
+    if (!boxed) {
+      for (int t = lane; t < WBOX; t += 64) box[t] = T(0);
+      boxed = true;
+    }
     const int b[3] = {q.x, q.y, q.z};
     T w[3][4], dw[3][4];
     const double fr[3] = {(double)f4.x, (double)f4.y, (double)f4.z};
@@ -678,6 +701,7 @@ __global__ __launch_bounds__(64) void adj_step_k(const T* __restrict__ phi0, con
         if (!(q.w & (1 << a))) hs[a] = h0[a] + (T)(-P.c[a]) * g * G[a];
     }
   }
+  if (!boxed) return;
   for (int t = lane; t < WBOX; t += 64) {
     const T v = box[t];
     if (v == T(0)) continue;
@@ -690,68 +714,166 @@ __global__ __launch_bounds__(64) void adj_step_k(const T* __restrict__ phi0, con
 
 // dL/dvel += the velocity scatter of the accumulated sensitivities H = hsum
 // (the tail of sl_adjoint_k: the MAC corners at the midpoint and, through the
-// midpoint's dependence on the node velocity, the node's faces), 16 x 4 x 4
-// blocks for the same lane combining.
-template <typename T, int BT>
-__global__ __launch_bounds__(256) void adj_finish_k(const T* __restrict__ vel, const T* __restrict__ hsum,
-                                                    T* __restrict__ gvel, AdjP P) {
-  const int tid = threadIdx.x + ABX * (threadIdx.y + ABY * threadIdx.z);
-  const int i = blockIdx.x * ABX + threadIdx.x, j = blockIdx.y * ABY + threadIdx.y, k = blockIdx.z * ABZ + threadIdx.z;
+// midpoint's dependence on the node velocity, the node's faces).  One wave
+// per block walks PZ planes of a 16 x 4 column and adds into a wave-private
+// LDS box of gvel (the column plus 1 node below and 2 above, all a midpoint
+// less than a cell away reaches) with plain read-add-write, as adj_step_k
+// does: lanes whose (x, y) corners of a component coincide are found with a
+// tag table and take LDS atomics, x-neighbour lanes hand shared corners to
+// the upper one, and a midpoint's corners beyond the box go to HBM with
+// atomics.  The box is laid out as gvel, so its flush is whole lines of
+// atomics, about 9 per node; the 30 contributions of a node each with its
+// own HBM atomic were what this kernel cost. 128^3
+// FP32, the 40% of the nodes that ten steps from the interface have reached:
+// 234 -> 59 us.
+constexpr int FBX = ABX + 3, FBY = ABY + 3;
+
+template <typename T, int BT, int PZ>
+__global__ __launch_bounds__(64) void adj_finish_k(const T* __restrict__ vel, const T* __restrict__ hsum,
+                                                   T* __restrict__ gvel, AdjP P) {
+  constexpr int FBZ = PZ + 3, FBOX = FBX * FBY * FBZ * 3;
+  __shared__ T box_s[FBOX];
+  __shared__ int tag_s[BT == DCL_RK2 ? 3 * FBX * FBY : 1];
+  typedef __attribute__((address_space(3))) T lds_T;
+  typedef __attribute__((address_space(3))) int lds_int;
+  volatile lds_T* box = (volatile lds_T*)box_s;
+  volatile lds_int* tag = (volatile lds_int*)tag_s;
+  constexpr int BSX = 3, BSY = 3 * FBX, BSZ = 3 * FBX * FBY;  // box strides
+  const int lane = threadIdx.x;
+  const int ox = blockIdx.x * ABX, oy = blockIdx.y * ABY, oz = blockIdx.z * PZ;
+  const int i = ox + (lane & (ABX - 1)), j = oy + lane / ABX;
   const int nx = P.w.nx, ny = P.w.ny, nz = P.w.nz;
-  const bool inner = i < nx && j < ny && k < nz && i >= 2 && i <= nx - 3 && j >= 2 && j <= ny - 3 && k >= 2 &&
-                     k <= nz - 3;
-  T H[3] = {T(0), T(0), T(0)};
-  if (inner) {
-    const T* hs = hsum + 3 * (int64_t)((k * ny + j) * nx + i);
-    H[0] = hs[0];
-    H[1] = hs[1];
-    H[2] = hs[2];
-  }
-  const bool act = inner && (H[0] != T(0) || H[1] != T(0) || H[2] != T(0));
-  T H1[3] = {T(0), T(0), T(0)};
-  MacState<T> m2;
-  if (act) {
+  const int sx = P.v.dof, sy = nx * P.v.dof, sz = ny * sy;
+  const bool in_xy = i >= 2 && i <= nx - 3 && j >= 2 && j <= ny - 3;
+  auto load_h = [&](int k, T (&H)[3]) {
+    H[0] = H[1] = H[2] = T(0);
+    if (in_xy && k >= 2 && k <= nz - 3 && k < oz + PZ) {
+      const T* hs = hsum + 3 * (int64_t)((k * ny + j) * nx + i);
+#pragma unroll
+      for (int a = 0; a < 3; ++a) H[a] = hs[a];
+    }
+  };
+  bool boxed = false;  // the box is in use (uniform)
+  T nH[3];
+  load_h(oz, nH);
+#pragma unroll 1
+  for (int k = oz; k < oz + PZ; ++k) {
+    const T H[3] = {nH[0], nH[1], nH[2]};
+    load_h(k + 1, nH);
+    const bool act = H[0] != T(0) || H[1] != T(0) || H[2] != T(0);  // interior nodes only
+    if (__ballot(act) == 0ull) continue;
+    if (!boxed) {
+      for (int t = lane; t < FBOX; t += 64) box[t] = T(0);
+      boxed = true;
+    }
+    T H1[3] = {T(0), T(0), T(0)};
     if (BT == DCL_RK2) {
-      const int X = P.w.px + i, Yg = P.w.py + j, Zg = P.w.pz + k;
-      const double Xd[3] = {(double)X, (double)Yg, (double)Zg};
-      T V1[3];
-      node_vel<T, 3>(vel, P.v, X, Yg, Zg, V1);
-      double Xm[3];
+      MacState<T> m;
+      if (act) {
+        const int X = P.w.px + i, Yg = P.w.py + j, Zg = P.w.pz + k;
+        const double Xd[3] = {(double)X, (double)Yg, (double)Zg};
+        T V1[3];
+        node_vel<T, 3>(vel, P.v, X, Yg, Zg, V1);
+        double Xm[3];
 #pragma unroll
-      for (int a = 0; a < 3; ++a) Xm[a] = Xd[a] - (double)V1[a] * P.ch[a];
-      bool cm[3] = {false, false, false};
-      mac_state<T>(vel, P.v, Xm, m2, cm);
+        for (int a = 0; a < 3; ++a) Xm[a] = Xd[a] - (double)V1[a] * P.ch[a];
+        bool cm[3] = {false, false, false};
+        mac_state<T>(vel, P.v, Xm, m, cm);
 #pragma unroll
-      for (int bb = 0; bb < 3; ++bb) {
-        const T K = H[0] * m2.dV[0][bb] + H[1] * m2.dV[1][bb] + H[2] * m2.dV[2][bb];
-        H1[bb] = (T)(-P.ch[bb]) * K;
+        for (int bb = 0; bb < 3; ++bb) {
+          const T K = H[0] * m.dV[0][bb] + H[1] * m.dV[1][bb] + H[2] * m.dV[2][bb];
+          H1[bb] = (T)(-P.ch[bb]) * K;
+        }
+      }
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        // the component's corner cube, in the box or not
+        const int bx = act ? m.bi[c][0] - (ox - 1) : 0, by = act ? m.bi[c][1] - (oy - 1) : 0,
+                  bz = act ? m.bi[c][2] - (oz - 1) : 0;
+        const bool on = act && H[c] != T(0);
+        const bool in_box = on && bx >= 0 && bx <= FBX - 2 && by >= 0 && by <= FBY - 2 && bz >= 0 && bz <= FBZ - 2;
+        const int slot = c * FBX * FBY + (in_box ? by * FBX + bx : 0);
+        if (in_box) tag[slot] = lane;
+        const bool lost = in_box && tag[slot] != lane;
+        if (lost) tag[slot] = -1;
+        const bool shared = in_box && tag[slot] == -1;
+        const bool plain = in_box && !shared;
+        const int key = in_box ? (bz * FBY + by) * FBX + bx + 1 : 0;
+        const int kl = lane_from_lower(key, 1), ku = lane_from_upper(key, 1);
+        const bool lo = in_box && kl != 0 && kl + 1 == key, up = in_box && ku != 0 && key + 1 == ku;
+        T a[4] = {T(0), T(0), T(0), T(0)}, b[4] = {T(0), T(0), T(0), T(0)};  // x0 / x1: y0z0 y1z0 y0z1 y1z1
+        if (on) {
+          const T x1 = m.f[c][0], x0 = T(1) - x1, y1 = m.f[c][1], y0 = T(1) - y1, z1 = m.f[c][2], z0 = T(1) - z1;
+          const T h = H[c];
+          a[0] = h * x0 * y0 * z0;
+          b[0] = h * x1 * y0 * z0;
+          a[1] = h * x0 * y1 * z0;
+          b[1] = h * x1 * y1 * z0;
+          a[2] = h * x0 * y0 * z1;
+          b[2] = h * x1 * y0 * z1;
+          a[3] = h * x0 * y1 * z1;
+          b[3] = h * x1 * y1 * z1;
+        }
+        if (on && !in_box) {
+          T* p = gvel + m.base[c];
+          const int off[4] = {0, sy, sz, sz + sy};
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            atomic_add(p + off[q], a[q]);
+            atomic_add(p + off[q] + sx, b[q]);
+          }
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const T bl = lane_from_lower(b[q], 1);
+          a[q] = lo ? a[q] + bl : a[q];
+        }
+        const int wo = bz * BSZ + by * BSY + bx * BSX + c;
+        // the two planes of one (x, y) corner together
+#pragma unroll
+        for (int y = 0; y < 2; ++y)
+#pragma unroll
+          for (int x = 0; x < 2; ++x) {
+            const int w0 = wo + y * BSY + x * BSX, w1 = w0 + BSZ;
+            const T v0 = x ? b[y] : a[y], v1 = x ? b[y + 2] : a[y + 2];
+            const bool mine = x == 0 || !up;
+            if (plain && mine) {
+              const T q0 = box[w0], q1 = box[w1];
+              box[w0] = q0 + v0;
+              box[w1] = q1 + v1;
+            }
+            if (shared && mine) {
+              atomicAdd(&box_s[w0], v0);
+              atomicAdd(&box_s[w1], v1);
+            }
+          }
       }
     } else {
 #pragma unroll
       for (int a = 0; a < 3; ++a) H1[a] = H[a];
     }
+    // node velocity: V_a = (f(X) + f(X + e_a)) / 2, each lane's words its own
+    const int no = (k - (oz - 1)) * BSZ + (j - (oy - 1)) * BSY + (i - (ox - 1)) * BSX;
+    if (act) {
+#pragma unroll
+      for (int a = 0; a < 3; ++a) {
+        const T h = T(0.5) * H1[a];
+        const int up1 = a == 0 ? BSX : a == 1 ? BSY : BSZ;
+        const T q0 = box[no + a];
+        box[no + a] = q0 + h;
+        const T q1 = box[no + a + up1];
+        box[no + a + up1] = q1 + h;
+      }
+    }
   }
-  if (BT == DCL_RK2) mac_scatter_lanes<T>(gvel, P.v, m2, H, act);
-  const int sx = P.v.dof, sy = P.w.nx * P.v.dof, sz = P.w.ny * sy;
-  const int gofs = (k * P.w.ny + j) * sy + i * sx + P.v.udof;
-  const T h0 = T(0.5) * H1[0], h1 = T(0.5) * H1[1], h2 = T(0.5) * H1[2];
-  const int nkey = act ? gofs + 1 : 0;
-  const int nkl = lane_from_lower(nkey, 1), nku = lane_from_upper(nkey, 1);
-  const bool nlo = act && nkl != 0 && nkl + sx == nkey, nup = act && nku != 0 && nkey + sx == nku;
-  const T h0l = lane_from_lower(h0, 1);
-  const int lane = tid & 63;
-  const int ykl = __shfl_up(nkey, ABX), yku = __shfl_down(nkey, ABX);
-  const bool ylo = act && lane >= ABX && ykl != 0 && ykl + sy == nkey;
-  const bool yup = act && lane < 64 - ABX && yku != 0 && nkey + sy == yku;
-  const T h1l = __shfl_up(h1, ABX);
-  if (act) {
-    T* gb = gvel + gofs;
-    atomic_add(gb, nlo ? h0 + h0l : h0);
-    if (!nup) atomic_add(gb + sx, h0);
-    atomic_add(gb + 1, ylo ? h1 + h1l : h1);
-    if (!yup) atomic_add(gb + sy + 1, h1);
-    atomic_add(gb + 2, h2);
-    atomic_add(gb + sz + 2, h2);
+  if (!boxed) return;
+  // flush the box: one HBM atomic per nonzero word (all of them in the window)
+  for (int t = lane; t < FBOX; t += 64) {
+    const T v = box[t];
+    if (v == T(0)) continue;
+    const int c = t % 3, r = t / 3;
+    const int lx = r % FBX, ly = (r / FBX) % FBY, lz = r / (FBX * FBY);
+    atomic_add(&gvel[(oz - 1 + lz) * sz + (oy - 1 + ly) * sy + (ox - 1 + lx) * sx + P.v.udof + c], v);
   }
 }
 
@@ -839,20 +961,37 @@ extern "C" int dcl_sl_adjoint_prepare(const dcl_window* win, const dcl_velocity*
   return adj_prepare_t<float>(interp, backtrace, vel->data, P, record, s);
 }
 
+static dim3 adj_grid(const KWin& w, int pz) {
+  return dim3((w.nx + ABX - 1) / ABX, (w.ny + ABY - 1) / ABY, (w.nz + pz - 1) / pz);
+}
+
+// Planes per wave of adj_step_k and adj_finish_k: 4, whose boxes hold fewer
+// words per node (8 were slower: 117 -> 131 us per 128^3 FP32 step), or 1
+// where 4 would leave a SIMD fewer than 4 waves and a wave's own latency is
+// the time.  Step / finish in us with 4 and with 1, gradient at the interface
+// only: 64^3 FP32 27 / 23 and 19 / 12, 80^3 FP64 34 / 24 and 23 / 14; gradient
+// everywhere: 128^3 FP32 118 / 107 and 182 / 130.
+static int adj_planes(const KWin& w) {
+  const dim3 g = adj_grid(w, 4);
+  return (int64_t)g.x * g.y * g.z >= 16 * (int64_t)device_cus() ? 4 : 1;
+}
+
 template <typename T>
 static int adj_step_t(int interp, const void* phi0, const void* record, const void* lam_next, void* lam,
                       void* hsum, const AdjP& P, hipStream_t s) {
   const int64_t n = (int64_t)P.w.nx * P.w.ny * P.w.nz;
   const int4* rb = static_cast<const int4*>(record);
-  dim3 grid((P.w.nx + ABX - 1) / ABX, (P.w.ny + ABY - 1) / ABY, (P.w.nz + AWZ - 1) / AWZ);
   const T* p0 = static_cast<const T*>(phi0);
   const T* ln = static_cast<const T*>(lam_next);
-  if (interp == DCL_CUBIC)
-    hipLaunchKernelGGL((adj_step_k<T, DCL_CUBIC>), grid, dim3(64), 0, s, p0, rb,
-                       static_cast<const void*>(rb + n), ln, static_cast<T*>(lam), static_cast<T*>(hsum), P);
-  else
-    hipLaunchKernelGGL((adj_step_k<T, DCL_LINEAR>), grid, dim3(64), 0, s, p0, rb,
-                       static_cast<const void*>(rb + n), ln, static_cast<T*>(lam), static_cast<T*>(hsum), P);
+#define DCL_STEP(I, PZ)                                                                                  \
+  hipLaunchKernelGGL((adj_step_k<T, I, PZ>), adj_grid(P.w, PZ), dim3(64), 0, s, p0, rb,                  \
+                     static_cast<const void*>(rb + n), ln, static_cast<T*>(lam), static_cast<T*>(hsum), P)
+  if (adj_planes(P.w) == 4) {
+    if (interp == DCL_CUBIC) DCL_STEP(DCL_CUBIC, 4); else DCL_STEP(DCL_LINEAR, 4);
+  } else {
+    if (interp == DCL_CUBIC) DCL_STEP(DCL_CUBIC, 1); else DCL_STEP(DCL_LINEAR, 1);
+  }
+#undef DCL_STEP
   DCL_LAUNCHED("adj_step");
   return 0;
 }
@@ -890,16 +1029,18 @@ extern "C" int dcl_sl_adjoint_finish(const dcl_window* win, const dcl_velocity* 
   AdjP P;
   DCL_TRY(adj_params(win, vel, dt, P));
   if (gvel == vel->data || gvel == hsum) return set_error(DCL_ERR_ARG_WRONG, "gvel must not alias inputs");
-  dim3 grid((P.w.nx + ABX - 1) / ABX, (P.w.ny + ABY - 1) / ABY, (P.w.nz + ABZ - 1) / ABZ);
   hipStream_t s = as_stream(stream);
-#define DCL_FIN(T, B)                                                                                      \
-  hipLaunchKernelGGL((adj_finish_k<T, B>), grid, dim3(ABX, ABY, ABZ), 0, s, static_cast<const T*>(vel->data), \
+#define DCL_FIN(T, B, PZ)                                                                                       \
+  hipLaunchKernelGGL((adj_finish_k<T, B, PZ>), adj_grid(P.w, PZ), dim3(64), 0, s, static_cast<const T*>(vel->data), \
                      static_cast<const T*>(hsum), static_cast<T*>(gvel), P)
-  if (precision == DCL_F64) {
-    if (backtrace == DCL_RK2) DCL_FIN(double, DCL_RK2); else DCL_FIN(double, DCL_EULER);
+#define DCL_FIN2(T, PZ) \
+  if (backtrace == DCL_RK2) DCL_FIN(T, DCL_RK2, PZ); else DCL_FIN(T, DCL_EULER, PZ)
+  if (adj_planes(P.w) == 4) {
+    if (precision == DCL_F64) { DCL_FIN2(double, 4); } else { DCL_FIN2(float, 4); }
   } else {
-    if (backtrace == DCL_RK2) DCL_FIN(float, DCL_RK2); else DCL_FIN(float, DCL_EULER);
+    if (precision == DCL_F64) { DCL_FIN2(double, 1); } else { DCL_FIN2(float, 1); }
   }
+#undef DCL_FIN2
 #undef DCL_FIN
   DCL_LAUNCHED("adj_finish");
   return 0;

@@ -53,6 +53,61 @@ def test_adjoint_matches_oracle(dev, dtype, tol, interp, bt):
             assert np.linalg.norm(got - ref) <= 2e-3 * np.linalg.norm(ref)
 
 
+@pytest.mark.parametrize("dtype,tol", [(torch.float64, 1e-11), (torch.float32, 2e-5)])
+@pytest.mark.parametrize("interp,bt", [("cubic", "rk2"), ("linear", "euler")])
+@pytest.mark.parametrize("n,dof", [((17, 9, 6), 3), ((130, 97, 40), 4), ((131, 130, 66), 3)])
+def test_steady_adjoint_sparse_gradient(dev, dtype, tol, interp, bt, n, dof):
+    """The record-driven step and its finish on a gradient that is zero in
+    whole columns, planes and single nodes (outer layers included), with one
+    and with four planes per wave, converging departures and departures beyond
+    the boxes: the sums of the per-step adjoint kernel (the tolerances of the
+    steady adjoint against it: rounding of reordered sums)."""
+    rng = np.random.default_rng(sum(n))
+    h = 1.0 / (max(n) - 1)
+    win = D.GridWindow((2, -1, 3), n, (h, h, h))
+    shape = win.shape
+    phi0 = to_dev(rng.normal(size=shape), dtype)
+    z, y, x = np.indices(shape, dtype=float)
+    vel = np.full(shape + (dof,), np.nan)
+    for c, q in enumerate((x / n[0], y / n[1], z / n[2])):
+        vel[..., dof - 3 + c] = np.sin(9 * q) - 1.5 * (q - 0.4) + 0.1 * rng.normal(size=shape)
+    dvel = to_dev(np.nan_to_num(vel), dtype)
+    dt = 2.4 * h / np.nanmax(np.abs(vel))
+    g = rng.normal(size=shape) * (rng.random(shape) < 0.5)
+    g[:, : n[1] // 3] = 0
+    g[n[2] // 2:, :, : n[0] // 2] = 0
+    dg = to_dev(g, dtype)
+    lam = torch.zeros_like(phi0)
+    gvel = torch.zeros_like(dvel)
+    if dof == 3:
+        A.sl_adjoint(phi0, dvel, dg, win, dt, interp, bt, lam, gvel)
+        rec = A.adjoint_record(dvel, win, dt, interp, bt)
+        lam2, hsum = torch.zeros_like(lam), torch.zeros(3 * win.nodes, dtype=dtype, device=dev)
+        A.adjoint_step(phi0, rec, dg, win, dt, lam2, hsum, interp)
+        gvel2 = A.adjoint_finish(dvel, hsum, win, dt, torch.zeros_like(dvel), bt)
+    else:  # the same velocity inside the fluid's records, through the C ABI
+        import ctypes as C
+
+        from dcell_amd import _lib as L
+        from dcell_amd.levelset import BACKTRACE, INTERP, _p, precision_of, stream_handle
+        inner = dvel[..., 1:].contiguous()
+        ginner = torch.zeros_like(inner)
+        A.sl_adjoint(phi0, inner, dg, win, dt, interp, bt, lam, ginner)
+        V = L.Velocity(C.c_void_p(dvel.data_ptr()), win.c(), 4, 1)
+        prec = precision_of(phi0)
+        rec = torch.empty(48 * win.nodes, dtype=torch.uint8, device=dev)
+        L.call("dcl_sl_adjoint_prepare", C.byref(win.c()), C.byref(V), dt, prec, INTERP[interp], BACKTRACE[bt],
+               _p(rec), stream_handle())
+        lam2, hsum = torch.zeros_like(lam), torch.zeros(3 * win.nodes, dtype=dtype, device=dev)
+        A.adjoint_step(phi0, rec, dg, win, dt, lam2, hsum, interp)
+        L.call("dcl_sl_adjoint_finish", C.byref(win.c()), C.byref(V), _p(hsum), _p(gvel), dt, prec, BACKTRACE[bt],
+               stream_handle())
+        assert float(gvel[..., 0].abs().max()) == 0
+        gvel, gvel2 = ginner, gvel[..., 1:].contiguous()
+    assert rel_max(to_np(lam2), to_np(lam)) <= tol
+    assert rel_max(to_np(gvel2), to_np(gvel)) <= tol
+
+
 @pytest.mark.parametrize("interp,bt", [("cubic", "rk2"), ("linear", "euler")])
 def test_adjoint_rough_velocity(dev, interp, bt):
     """Velocity noise from node to node: x-neighbour stencils land 0, 1, 2, 3
