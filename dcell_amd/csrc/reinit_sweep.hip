@@ -62,7 +62,6 @@ struct RsCell {
   unsigned char* cd[2];  // per chunk of RS_CH nodes: it holds a mark in nd[k & 1]
   KWin w;
   int d3;
-  int small;  // below 2^28 nodes: buffer loads
   double bw, inf, tol;
   long long qb0, qb1;  // the level set's raster blocks (RS_B nodes each) in the batch
   long long cb0;       // its first chunk (RS_CH nodes) in the batch
@@ -101,11 +100,17 @@ __device__ __forceinline__ int rs_find(const RsCell* __restrict__ cells, int nce
 
 __device__ __forceinline__ int64_t rs_nodes(const RsCell& c) { return (int64_t)c.w.nx * c.w.ny * c.w.nz; }
 
+// A level set's arrays are named by a table in memory, so their pointers are
+// cast to the global address space (the compiler would take them for flat).
+template <typename T>
+using rs_gptr = __attribute__((address_space(1))) T*;
+
 // a node changed: the nodes whose stencil holds it (itself and two nodes
 // each way along each axis) are recomputed in the next sweep
 template <int DIM>
-__device__ __forceinline__ void rs_mark(const RsCell& c, unsigned char* nd, unsigned char* cd, int64_t i, int lx,
+__device__ __forceinline__ void rs_mark(const RsCell& c, unsigned char* nd_, unsigned char* cd_, int64_t i, int lx,
                                         int ly, int lz) {
+  const rs_gptr<unsigned char> nd = (rs_gptr<unsigned char>)nd_, cd = (rs_gptr<unsigned char>)cd_;
   const int64_t sy = c.w.nx, sz = (int64_t)c.w.nx * c.w.ny;
   nd[i] = 1;
   cd[i / RS_CH] = 1;
@@ -170,124 +175,97 @@ __global__ __launch_bounds__(RS_B) void rs_bc_k(const RsCell* __restrict__ cells
   rs_mark<DIM>(c, c.nd[0], c.cd[0], j, n.pos.x - c.w.px, n.pos.y - c.w.py, c.d3 ? n.pos.z - c.w.pz : 0);
 }
 
-// a byte or a double of a level set's node array (buffer loads below 2^28
-// nodes)
-__device__ __forceinline__ unsigned rs_byte(const RsCell& c, const unsigned char* p, int64_t i) {
-  if (c.small) return __builtin_amdgcn_raw_buffer_load_b8(make_rsrc(p, (unsigned)rs_nodes(c)), (int)i, 0, 0);
-  return p[i];
-}
-
-__device__ __forceinline__ double rs_f64(const RsCell& c, const double* p, int64_t i) {
-  if (c.small) return BL<double>::one(make_rsrc(p, (unsigned)(8 * rs_nodes(c))), (int)(8 * i), 0);
-  return p[i];
-}
-
-// a neighbour as the side `sign` sees it: its value q = sign * phi, the time
-// it is accepted (-1: before the side's pops, its value for a node of this
-// side, INFINITY: never) and whether it pushes its neighbours in this side
-struct RsNb {
-  double q, t;
-  bool push;
-};
-
-__device__ __forceinline__ RsNb rs_view(double inf, int sign, double v, int m) {
-  RsNb r;
-  r.q = inf;
-  r.t = INFINITY;
-  r.push = false;
-  if (m == RS_OUT) return r;
-  const double q = sign * v;
-  r.q = q;
-  if (m == 2) {
-    // a boundary node pushes in this side when sign * phi >= 0
-    if (0 <= q && q < inf) {
-      r.t = -1;
-      r.push = true;
-    }
-  } else if (m == (sign > 0 ? 1 : 0)) {
-    if (q < inf) {
-      r.t = q;
-      r.push = true;
-    }
-  } else if (sign > 0 && 0 <= q && q < inf) {
-    r.t = -1;  // a - side node: final before the + side starts
-  }
-  return r;
-}
-
-// the acceptance-time code of a neighbour as the side `sign` sees it (see
-// rs_view): its time, or RS_T_STATIC for a node accepted from the start that
-// does not push in this side
+// The acceptance-time code of a neighbour of value v and mask m as the side
+// `sign` sees it, q = sign * v: its value for an accepted node of this side,
+// which pushes its neighbours at that time; -1 for a boundary node with q >= 0,
+// which pushes before the side's pops; RS_T_STATIC for a - side node that the
+// + side finds final, which does not push; INFINITY for a node never accepted.
 constexpr double RS_T_STATIC = -2.0;
 
 __device__ __forceinline__ double rs_tcode(double inf, int sign, double v, int m) {
-  const RsNb n = rs_view(inf, sign, v, m);
-  return n.push ? n.t : (n.t < INFINITY ? RS_T_STATIC : INFINITY);
+  const double q = sign * v;
+  const bool own = m == (sign > 0 ? 1 : 0), bc = m == 2, other = (sign > 0) & (m == 0);
+  const bool known = (q < inf) & (own | ((0 <= q) & (bc | other)));
+  const double t = own ? q : bc ? -1.0 : RS_T_STATIC;
+  return known ? t : INFINITY;
+}
+
+// One direction of an axis as a node's pushes see it: AccumulateCoef's
+// (FastMarching2D.c:33-94) differences from the node, which is not accepted
+// and counts as inf, to its neighbour (value p) and the node beyond it.  The
+// terms depend on the acceptances only through which of the two hold, so
+// they are formed once; a push at time T takes the second-order ones from e2
+// on, the first-order ones from e1 on.
+struct RsSide {
+  double p, q;    // the neighbour's value; (4 p - beyond) / 3
+  double D2;      // the second-order difference
+  double e1, e2;  // the times from which each order holds (INFINITY: never)
+};
+
+// t1, t2: the acceptance-time codes of the neighbour and the node beyond
+__device__ __forceinline__ RsSide rs_side(double inf, double p, double t1, double beyond, double t2) {
+#pragma clang fp contract(off)
+  RsSide s;
+  s.p = p;
+  s.q = (4 * p - beyond) / 3;
+  s.D2 = (3 * inf - 4 * p + beyond) / 2.;
+  const bool first = (0 <= p) & (p < inf);  // inf - p > 0
+  const bool second = first & (0 <= beyond) & (beyond < inf) & (s.D2 > 0);
+  s.e1 = first ? t1 : INFINITY;
+  s.e2 = second ? fmax(t1, t2) : INFINITY;
+  return s;
 }
 
 // the node's value from its stencil: nv the values and nt the
 // acceptance-time codes (for the node's side) of the nodes two each way
-// along each axis (-2, -1, +1, +2); NaN for a NaN update.  An axis's
-// AccumulateCoef terms depend only on which of its four nodes are accepted,
-// so they are kept from one push to the next and recomputed when that
-// changes; the sums over the axes are redone in axis order each push (no
-// partial sum is ever -0, so adding a kept term gives the same bits as
-// adding it fresh).
+// along each axis (-2, -1, +1, +2); NaN for a NaN update.  Each push takes
+// the larger difference of each axis's two directions (the + one when
+// equal), sums the terms in axis order and solves the quadratic; the larger
+// root's numerator falls back to -B where the discriminant is negative.
 template <int DIM>
 __device__ __forceinline__ double rs_node(double inf, double bw, int sign, const double (&nv)[DIM][4],
                                           const double (&nt)[DIM][4]) {
 #pragma clang fp contract(off)
-  double cand = INFINITY, last = -INFINITY;
-  double ta[DIM], tb[DIM], tc[DIM];
-  unsigned sig[DIM];
+  double cand = INFINITY;
+  RsSide sd[DIM][2];       // [axis][0: +, 1: -]
+  double push[DIM][2];     // push times not yet replayed
 #pragma unroll
   for (int a = 0; a < DIM; ++a) {
-    ta[a] = tb[a] = tc[a] = 0.0;
-    sig[a] = ~0u;
+    sd[a][0] = rs_side(inf, sign * nv[a][2], nt[a][2], sign * nv[a][3], nt[a][3]);
+    sd[a][1] = rs_side(inf, sign * nv[a][1], nt[a][1], sign * nv[a][0], nt[a][0]);
+    push[a][0] = nt[a][2] == RS_T_STATIC ? INFINITY : nt[a][2];
+    push[a][1] = nt[a][1] == RS_T_STATIC ? INFINITY : nt[a][1];
   }
   // at most 2 * DIM distinct push times, then one pass that finds none
 #pragma unroll 1
   for (int guard = 0; guard <= 2 * DIM; ++guard) {
     double T = INFINITY;
 #pragma unroll
-    for (int a = 0; a < DIM; ++a)
-#pragma unroll
-      for (int k = 1; k <= 2; ++k) {
-        const double t = nt[a][k];
-        if (t != RS_T_STATIC && t > last && t < T) T = t;
-      }
+    for (int a = 0; a < DIM; ++a) T = fmin(T, fmin(push[a][0], push[a][1]));
     if (T == INFINITY || !(T < cand)) break;
-#pragma unroll
-    for (int a = 0; a < DIM; ++a) {
-      unsigned sg = 0;
-#pragma unroll
-      for (int k = 0; k < 4; ++k) sg |= nt[a][k] <= T ? 1u << k : 0u;
-      if (sg != sig[a]) {
-        sig[a] = sg;
-        double loc[7];
-        loc[0] = loc[6] = loc[3] = inf;
-#pragma unroll
-        for (int k = 0; k < 4; ++k) loc[k < 2 ? k + 1 : k + 2] = (sg >> k) & 1u ? sign * nv[a][k] : inf;
-        double x = 0, y = 0, z = 0;
-        ri_accumulate(inf, loc, x, y, z);
-        ta[a] = x;
-        tb[a] = y;
-        tc[a] = z;
-      }
-    }
     double A = 0, B = 0, C = -1;
 #pragma unroll
     for (int a = 0; a < DIM; ++a) {
-      A += ta[a];
-      B += tb[a];
-      C += tc[a];
+      const RsSide &sp = sd[a][0], &sm = sd[a][1];
+      const bool p1 = sp.e1 <= T, p2 = sp.e2 <= T, m1 = sm.e1 <= T, m2 = sm.e2 <= T;
+      const double Dp = p2 ? sp.D2 : p1 ? inf - sp.p : 0.0;
+      const double Dm = m2 ? sm.D2 : m1 ? inf - sm.p : 0.0;
+      const bool minus = Dm > Dp;
+      const bool second = minus ? m2 : p2, first = minus ? m1 : p1;
+      const double x = minus ? (m2 ? sm.q : sm.p) : (p2 ? sp.q : sp.p);
+      // 9/4, -9/2 x, 9/4 x x; or 1, -2 x, x x; or nothing
+      const double ka = second ? 9. / 4. : 1., kb = second ? -9. / 2. : -2.;
+      const bool some = first | second;
+      A += some ? ka : 0.;
+      B += some ? kb * x : 0.;
+      C += some ? ka * x * x : 0.;
+#pragma unroll
+      for (int d = 0; d < 2; ++d) push[a][d] = push[a][d] <= T ? INFINITY : push[a][d];
     }
     const double disc = sqrt(B * B - 4 * A * C);
-    double d1 = (-B + disc) / (2 * A);
-    if (d1 != d1) d1 = -B / (2 * A);
+    const double d1 = (disc != disc ? -B : -B + disc) / (2 * A);
     if (d1 != d1) return NAN;
     if (d1 < cand) cand = d1;
-    last = T;
   }
   return cand <= bw ? sign * cand : sign * inf;
 }
@@ -357,10 +335,7 @@ __global__ __launch_bounds__(RS_B) void rs_need_k(const RsCell* __restrict__ cel
       unsigned w = 0;
       if (i0 < n) {
         // the mark arrays are padded to 256 bytes, so a whole word is in them
-        if (c.small)
-          w = __builtin_amdgcn_raw_buffer_load_b32(make_rsrc(nd, (unsigned)((n + 3) & ~3ll)), (int)i0, 0, 0);
-        else
-          w = *reinterpret_cast<const unsigned*>(nd + i0);
+        w = *(rs_gptr<const unsigned>)(nd + i0);
         if (i0 + 4 > n) w &= n - i0 == 1 ? 0xffu : n - i0 == 2 ? 0xffffu : 0xffffffu;
         if (w) *reinterpret_cast<unsigned*>(nd + i0) = 0u;
       }
@@ -381,64 +356,82 @@ __global__ __launch_bounds__(RS_B) void rs_need_k(const RsCell* __restrict__ cel
   }
 }
 
-// the listed nodes' new values, one thread each.  The per-sweep counts of
-// moving nodes are added into nparts partial sums per level set, each on
-// its own 128-byte line (part p of level set i at p * pstride + i).
+// the listed nodes' new values, one thread each.  A wave works its nodes of
+// one level set at a time (nearly always all of them), so that the level
+// set's arrays are the same for the lanes at work, and every load of a node's
+// stencil is issued before the first is waited for: nodes outside the window
+// load the node itself instead.  At 256^3 with 600 000 listed nodes 71 -> 37 us
+// against a level set per lane (a loop over its values around every load) and
+// the terms of each axis formed anew at every push.  Three waves per SIMD: at
+// 168 registers nothing spills; two (173) took 6% more per reinitialisation,
+// four spilled and took 18% more.  The per-sweep counts of moving nodes are
+// added into nparts partial sums per level set, each on its own 128-byte
+// line (part p of level set i at p * pstride + i).
 template <int DIM>
-__global__ __launch_bounds__(RS_B) void rs_update_k(const RsCell* __restrict__ cells, RsState* __restrict__ st,
+__device__ __forceinline__ bool rs_update_node(const RsCell& c, RsState* __restrict__ st, int64_t i) {
+#pragma clang fp contract(off)
+  const int k = st->k, settle = st->settle;
+  const rs_gptr<const double> in = (rs_gptr<const double>)((k & 1) ? c.buf[1] : c.buf[0]);
+  const rs_gptr<double> out = (rs_gptr<double>)((k & 1) ? c.buf[0] : c.buf[1]);
+  const rs_gptr<const unsigned char> mask = (rs_gptr<const unsigned char>)c.mask;
+  const int64_t sy = c.w.nx, sz = (int64_t)c.w.nx * c.w.ny;
+  const int lz = DIM == 3 ? (int)((unsigned)i / (unsigned)sz) : 0;
+  const int r2 = (int)(i - lz * sz);
+  const int ly = (int)((unsigned)r2 / (unsigned)c.w.nx), lx = r2 - ly * c.w.nx;
+  double nv[DIM][4], nt[DIM][4];
+  int mm[DIM][4];
+  const int m = mask[i];
+  const double old = in[i];
+#pragma unroll
+  for (int a = 0; a < DIM; ++a) {
+    const int p = a == 0 ? lx : a == 1 ? ly : lz;
+    const int lim = a == 0 ? c.w.nx : a == 1 ? c.w.ny : c.w.nz;
+    const int64_t st_ = a == 0 ? 1 : a == 1 ? sy : sz;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int o = q < 2 ? q - 2 : q - 1;
+      const bool inside = (unsigned)(p + o) < (unsigned)lim;
+      const int64_t at = inside ? i + o * st_ : i;
+      nv[a][q] = in[at];
+      const int b = mask[at];
+      mm[a][q] = inside ? b : RS_OUT;
+    }
+  }
+  if (m == 2) return false;
+  const int sg = m ? 1 : -1;
+#pragma unroll
+  for (int a = 0; a < DIM; ++a)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) nt[a][q] = rs_tcode(c.inf, sg, nv[a][q], mm[a][q]);
+  const double u = rs_node<DIM>(c.inf, c.bw, sg, nv, nt);
+  if (u != u) atomicOr(&st->nan, 1);
+  double v = old;
+  if (!settle || sg * u < sg * v) v = u;
+  out[i] = v;
+  if (__double_as_longlong(v) != __double_as_longlong(old))
+    rs_mark<DIM>(c, (k & 1) ? c.nd[0] : c.nd[1], (k & 1) ? c.cd[0] : c.cd[1], i, lx, ly, lz);
+  return fabs(v - old) > c.tol;
+}
+
+template <int DIM>
+__global__ __launch_bounds__(RS_B) __attribute__((amdgpu_waves_per_eu(3, 8))) void rs_update_k(const RsCell* __restrict__ cells, RsState* __restrict__ st,
                                                     const int2* __restrict__ nlist, const int* __restrict__ ncount,
                                                     unsigned long long* __restrict__ parts, int nparts, int pstride) {
-#pragma clang fp contract(off)
   const int n = *ncount;
   for (int e0 = blockIdx.x * RS_B; e0 < n; e0 += gridDim.x * RS_B) {
     const int e = e0 + threadIdx.x;
     bool moved = false;
     int ci = -1;
+    int64_t i = 0;
     if (e < n) {
       const int2 w = nlist[e];
       ci = w.x;
-      const RsCell& c = cells[ci];
-      const int k = st[ci].k, settle = st[ci].settle;
-      const double* __restrict__ in = (k & 1) ? c.buf[1] : c.buf[0];
-      double* __restrict__ out = (k & 1) ? c.buf[0] : c.buf[1];
-      unsigned char* __restrict__ ncur = (k & 1) ? c.nd[0] : c.nd[1];
-      unsigned char* __restrict__ ccur = (k & 1) ? c.cd[0] : c.cd[1];
-      const int64_t i = w.y;
-      const int64_t sy = c.w.nx, sz = (int64_t)c.w.nx * c.w.ny;
-      const int lz = DIM == 3 ? (int)(i / sz) : 0;
-      const int r2 = (int)(i - lz * sz);
-      const int ly = r2 / c.w.nx, lx = r2 - ly * c.w.nx;
-      const int m = rs_byte(c, c.mask, i);
-      if (m != 2) {
-        const double old = rs_f64(c, in, i);
-        const int sg = m ? 1 : -1;
-        double nv[DIM][4], nt[DIM][4];
-#pragma unroll
-        for (int a = 0; a < DIM; ++a) {
-          const int p = a == 0 ? lx : a == 1 ? ly : lz;
-          const int lim = a == 0 ? c.w.nx : a == 1 ? c.w.ny : c.w.nz;
-          const int64_t st_ = a == 0 ? 1 : a == 1 ? sy : sz;
-#pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            const int o = q < 2 ? q - 2 : q - 1;
-            double v = 0.0;
-            int mm = RS_OUT;
-            if (p + o >= 0 && p + o < lim) {
-              v = rs_f64(c, in, i + o * st_);
-              mm = rs_byte(c, c.mask, i + o * st_);
-            }
-            nv[a][q] = v;
-            nt[a][q] = rs_tcode(c.inf, sg, v, mm);
-          }
-        }
-        const double u = rs_node<DIM>(c.inf, c.bw, sg, nv, nt);
-        if (u != u) atomicOr(&st[ci].nan, 1);
-        double v = old;
-        if (!settle || sg * u < sg * v) v = u;
-        moved = fabs(v - old) > c.tol;
-        out[i] = v;
-        if (__double_as_longlong(v) != __double_as_longlong(old)) rs_mark<DIM>(c, ncur, ccur, i, lx, ly, lz);
-      }
+      i = w.y;
+    }
+    for (unsigned long long todo = __ballot(ci >= 0); todo;) {
+      const int cu = __builtin_amdgcn_readlane(ci, __builtin_ctzll(todo));
+      if (ci == cu) moved = rs_update_node<DIM>(cells[cu], st + cu, i);
+      todo &= ~__ballot(ci == cu);
     }
     // one atomic per wave where the wave's nodes are of one level set
     const int c0 = __builtin_amdgcn_readfirstlane(ci);
@@ -781,7 +774,6 @@ extern "C" int dcl_reinitialize_parallel(dcl_reinit_cell* cells, int ncells, int
     c.cd[1] = reinterpret_cast<unsigned char*>(take((size_t)((n + RS_CH - 1) / RS_CH)));
     c.w = kwin(u.win);
     c.d3 = d3;
-    c.small = n < (1 << 28);
     c.bw = u.band_width;
     c.inf = u.phi_inf;
     c.tol = u.band_width * RS_TOL;
