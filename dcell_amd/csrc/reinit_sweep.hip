@@ -25,14 +25,15 @@
 // each sweep recomputes only the marked nodes; the output buffer already
 // holds the others' values (both buffers start equal, and a node not
 // recomputed did not change in the sweep before).  The boundary values are
-// the changes before the first sweep.  A sweep is three launches: one lists
+// the changes before the first sweep.  A sweep is two launches: one lists
 // the marked nodes (each chunk of 1024 nodes carries a flag set with its
 // marks, so a block reads its chunks' flags at once and scans only the
-// marked chunks, four marks per thread, clearing them), one updates the
-// listed nodes, one thread each, so that whole waves run the chain of
-// updates, and one wave per level set sums the moved nodes and decides.
-// Lists are gathered per block in LDS and published with one atomic each:
-// an atomic per wave on one counter would queue.
+// marked chunks, one wave each with 16 marks per lane, clearing them) and, in
+// blocks of its own, sums the moved nodes of the sweep before and decides;
+// the other updates the listed nodes, one thread each, so that whole waves
+// run the chain of updates.  Lists are gathered per block in LDS and
+// published with one atomic each: an atomic per wave on one counter would
+// queue (6 ns each).
 //
 // A batch of level sets runs in one launch per step, over all nodes (in
 // raster order) and all records, each block finding its level set by a
@@ -50,8 +51,11 @@ constexpr int RS_B = 256;
 constexpr double RS_TOL = 1e-9;  // settled: no node moves by more than band_width * RS_TOL
 constexpr int RS_OUT = 3;        // the mask of a stencil node outside the window
 constexpr int RS_CH = 1024;      // nodes per chunk of the mark scan (four per thread)
-constexpr int RS_STAGE = 2048;   // list entries a block gathers before publishing them
-constexpr int RS_NEED_GRID = 2048;  // blocks of the mark scan
+constexpr int RS_STAGE = 3072;   // list entries a block gathers before publishing them
+// blocks of the mark scan: each publishes its entries with an atomic on one
+// counter, and fewer leave waves idle (a 256^3 step with 512, 1024, 2048 and
+// 4096: 1.64, 1.60, 1.78 and 2.05 ms)
+constexpr int RS_NEED_GRID = 1024;
 constexpr int RS_GRID = 4096;       // blocks of the update, each taking listed nodes in turn
 constexpr int RS_GROUP = 4;         // sweeps queued between looks at the count of level sets still sweeping
 
@@ -104,6 +108,7 @@ __device__ __forceinline__ int64_t rs_nodes(const RsCell& c) { return (int64_t)c
 // cast to the global address space (the compiler would take them for flat).
 template <typename T>
 using rs_gptr = __attribute__((address_space(1))) T*;
+typedef unsigned rs_u32x4 __attribute__((ext_vector_type(4)));
 
 // a node changed: the nodes whose stencil holds it (itself and two nodes
 // each way along each axis) are recomputed in the next sweep
@@ -288,72 +293,140 @@ __device__ __forceinline__ int rs_scan(int v, unsigned* wsum, int* total) {
   return pre + x - v;
 }
 
-// the nodes a sweep recomputes: the marked ones, read and cleared four at a
-// time (the marks of the sweep after next are written into these bytes)
+// after a sweep, one wave per level set: the count of moving nodes decides
+// whether it has settled and whether its values may only go down from the
+// next sweep on.  active: the level sets still sweeping.
+__device__ __forceinline__ void rs_state_of(RsState* __restrict__ st, int i, int max_sweeps, int* __restrict__ active,
+                                            unsigned long long* __restrict__ parts, int nparts, int pstride) {
+  const int lane = threadIdx.x & 63;
+  if (st[i].done) return;
+  unsigned long long c = 0;
+  if (lane < nparts) {
+    c = parts[(long long)lane * pstride + i];
+    parts[(long long)lane * pstride + i] = 0;
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o, 64);
+  if (lane != 0) return;
+  RsState s = st[i];
+  s.k++;
+  if (s.nan) {
+    s.done = RS_NAN;
+  } else if (c == 0) {
+    s.done = RS_SETTLED;
+  } else {
+    if (s.last >= 0 && (long long)c < s.last) s.falling = 1;
+    else if (s.last >= 0 && s.falling) s.settle = 1;
+    s.last = (long long)c;
+    if (s.k >= max_sweeps) s.done = RS_SWEEPS;
+  }
+  st[i] = s;
+  if (!s.done) atomicAdd(active, 1);
+}
+
+// The nodes sweep `sweep` recomputes: the marked ones, read and cleared 16 at
+// a time (the marks of the sweep after next are written into these bytes).
+// One wave per marked chunk; a block's entries are gathered in LDS and
+// published with one atomic, entries past the LDS space with one per chunk.
+// The last nstate blocks step the level sets' states after the sweep before
+// (sweep > 0), which the next update needs and the mark scan does not: which
+// marks a sweep reads depends on its number alone, and a level set settled
+// just now only lists nodes that the update then leaves out.
 __global__ __launch_bounds__(RS_B) void rs_need_k(const RsCell* __restrict__ cells, int ncells,
-                                                  const RsState* __restrict__ st, long long nch,
-                                                  int2* __restrict__ nlist, int* __restrict__ ncount) {
+                                                  RsState* __restrict__ st, long long nch, int sweep, int scan_blocks,
+                                                  int2* __restrict__ nlist, int* __restrict__ ncount, int max_sweeps,
+                                                  int* __restrict__ active, unsigned long long* __restrict__ parts,
+                                                  int nparts, int pstride) {
   __shared__ int2 stage[RS_STAGE];
   __shared__ unsigned wsum[RS_B / 64];
-  __shared__ int at;
+  __shared__ int at, held, cut;  // entries reserved; the first reservation past the LDS space
   __shared__ int live[RS_B];  // this round's chunks holding marks, as batch chunk indices
-  const int tid = threadIdx.x;
-  int held = 0;  // entries in stage (uniform)
-  // the block's chunks are blockIdx.x + q * gridDim.x; their flags are read
-  // RS_B at a time, one per thread, and the marked ones visited in turn
-  const long long per = (nch - blockIdx.x + gridDim.x - 1) / gridDim.x;
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  if ((int)blockIdx.x >= scan_blocks) {
+    const int i = ((int)blockIdx.x - scan_blocks) * (RS_B / 64) + wv;
+    if (i < ncells) rs_state_of(st, i, max_sweeps, active, parts, nparts, pstride);
+    return;
+  }
+  if (tid == 0) {
+    held = 0;
+    cut = RS_STAGE;
+  }
+  // the block's chunks are blockIdx.x + q * scan_blocks; their flags are read
+  // RS_B at a time, one per thread, and the marked ones taken by the waves in
+  // turn
+  const long long per = (nch - blockIdx.x + scan_blocks - 1) / scan_blocks;
   for (long long q0 = 0; q0 < per; q0 += RS_B) {
-    const long long g = blockIdx.x + (q0 + tid) * gridDim.x;
+    const long long g = blockIdx.x + (q0 + tid) * scan_blocks;
     bool has = false;
     if (q0 + tid < per) {
       const int ci = rs_find<RS_KEY_CHUNK>(cells, ncells, g);
       const RsCell& c = cells[ci];
-      if (!st[ci].done) {
-        unsigned char* cdk = (st[ci].k & 1) ? c.cd[1] : c.cd[0];
-        has = cdk[g - c.cb0] != 0;
-        if (has) cdk[g - c.cb0] = 0;
-      }
+      const rs_gptr<unsigned char> cdk = (rs_gptr<unsigned char>)c.cd[sweep & 1];
+      has = cdk[g - c.cb0] != 0;
+      if (has) cdk[g - c.cb0] = 0;
     }
     int nlive;
     const int slot = rs_scan(has ? 1 : 0, wsum, &nlive);
     if (has) live[slot] = (int)g;
     __syncthreads();
-    for (int e = 0; e < nlive; ++e) {
-      if (held + RS_CH > RS_STAGE) {
-        if (tid == 0) at = atomicAdd(ncount, held);
-        __syncthreads();
-        for (int q = tid; q < held; q += RS_B) nlist[at + q] = stage[q];
-        __syncthreads();
-        held = 0;
-      }
+    for (int e = wv; e < nlive; e += RS_B / 64) {
       const long long gc = live[e];
-      const int ci = rs_find<RS_KEY_CHUNK>(cells, ncells, gc);
+      const int ci = __builtin_amdgcn_readfirstlane(rs_find<RS_KEY_CHUNK>(cells, ncells, gc));
       const RsCell& c = cells[ci];
-      unsigned char* nd = (st[ci].k & 1) ? c.nd[1] : c.nd[0];
       const int64_t n = rs_nodes(c);
-      const int64_t i0 = (gc - c.cb0) * RS_CH + 4 * tid;
-      unsigned w = 0;
-      if (i0 < n) {
-        // the mark arrays are padded to 256 bytes, so a whole word is in them
-        w = *(rs_gptr<const unsigned>)(nd + i0);
-        if (i0 + 4 > n) w &= n - i0 == 1 ? 0xffu : n - i0 == 2 ? 0xffffu : 0xffffffu;
-        if (w) *reinterpret_cast<unsigned*>(nd + i0) = 0u;
-      }
-      const int cnt = ((w & 0xffu) != 0) + ((w & 0xff00u) != 0) + ((w & 0xff0000u) != 0) + ((w >> 24) != 0);
-      int tot;
-      int pos = held + rs_scan(cnt, wsum, &tot);
+      const int64_t i0 = (gc - c.cb0) * RS_CH + 16 * lane;
+      // the mark arrays are padded to 256 bytes
+      const rs_gptr<rs_u32x4> nd = (rs_gptr<rs_u32x4>)(c.nd[sweep & 1] + i0);
+      rs_u32x4 w = {0u, 0u, 0u, 0u};
+      if (i0 < n) w = *nd;
+      // marks are 0 or 1 per byte: bit j of m = byte j
+      unsigned m = 0;
 #pragma unroll
-      for (int b2 = 0; b2 < 4; ++b2)
-        if ((w >> (8 * b2)) & 0xffu) stage[pos++] = make_int2(ci, (int)(i0 + b2));
-      held += tot;
-      __syncthreads();
+      for (int j = 0; j < 4; ++j) m |= ((((w[j] & 0x01010101u) * 0x01020408u) >> 24) & 0xfu) << (4 * j);
+      if (i0 + 16 > n && i0 < n) m &= (1u << (int)(n - i0)) - 1u;
+      if (m) *nd = rs_u32x4{0u, 0u, 0u, 0u};
+      const int cnt = __popc(m);
+      int pre = cnt;
+#pragma unroll
+      for (int o = 1; o < 64; o <<= 1) {
+        const int t = __shfl_up(pre, o, 64);
+        if (lane >= o) pre += t;
+      }
+      const int tot = __shfl(pre, 63);
+      if (tot == 0) continue;
+      int base = 0;
+      if (lane == 63) base = atomicAdd(&held, tot);
+      base = __shfl(base, 63);
+      const bool fits = base + tot <= RS_STAGE;
+      if (!fits) {
+        if (lane == 63) {
+          atomicMin(&cut, base);
+          base = atomicAdd(ncount, tot);
+        }
+        base = __shfl(base, 63);
+      }
+      int pos = base + pre - cnt;
+      for (; m; m &= m - 1) {
+        const int2 ent = make_int2(ci, (int)(i0 + __ffs((int)m) - 1));
+        if (fits) stage[pos++] = ent;
+        else nlist[pos++] = ent;
+      }
     }
-  }
-  if (held > 0) {
-    if (tid == 0) at = atomicAdd(ncount, held);
     __syncthreads();
-    for (int q = tid; q < held; q += RS_B) nlist[at + q] = stage[q];
   }
+  const int n = min(held, cut);  // uniform: every reservation is made
+  if (n > 0) {
+    if (tid == 0) at = atomicAdd(ncount, n);
+    __syncthreads();
+    for (int q = tid; q < n; q += RS_B) nlist[at + q] = stage[q];
+  }
+}
+
+__global__ __launch_bounds__(RS_B) void rs_state_k(RsState* __restrict__ st, int ncells, int max_sweeps,
+                                                   int* __restrict__ active, unsigned long long* __restrict__ parts,
+                                                   int nparts, int pstride) {
+  const int i = blockIdx.x * (RS_B / 64) + (threadIdx.x >> 6);
+  if (i < ncells) rs_state_of(st, i, max_sweeps, active, parts, nparts, pstride);
 }
 
 // the listed nodes' new values, one thread each.  A wave works its nodes of
@@ -370,6 +443,7 @@ __global__ __launch_bounds__(RS_B) void rs_need_k(const RsCell* __restrict__ cel
 template <int DIM>
 __device__ __forceinline__ bool rs_update_node(const RsCell& c, RsState* __restrict__ st, int64_t i) {
 #pragma clang fp contract(off)
+  if (st->done) return false;
   const int k = st->k, settle = st->settle;
   const rs_gptr<const double> in = (rs_gptr<const double>)((k & 1) ? c.buf[1] : c.buf[0]);
   const rs_gptr<double> out = (rs_gptr<double>)((k & 1) ? c.buf[0] : c.buf[1]);
@@ -445,40 +519,6 @@ __global__ __launch_bounds__(RS_B) __attribute__((amdgpu_waves_per_eu(3, 8))) vo
       atomicAdd(&parts[(long long)((e0 / RS_B) % nparts) * pstride + ci], 1ull);
     }
   }
-}
-
-// after a sweep, one wave per level set: the count of moving nodes decides
-// whether it has settled and whether its values may only go down from the
-// next sweep on
-__global__ __launch_bounds__(RS_B) void rs_state_k(RsState* __restrict__ st, int ncells, int max_sweeps,
-                                                   int* __restrict__ active, unsigned long long* __restrict__ parts,
-                                                   int nparts, int pstride) {
-  const int i = blockIdx.x * (RS_B / 64) + (threadIdx.x >> 6);
-  const int lane = threadIdx.x & 63;
-  if (i >= ncells) return;
-  if (st[i].done) return;
-  unsigned long long c = 0;
-  if (lane < nparts) {
-    c = parts[(long long)lane * pstride + i];
-    parts[(long long)lane * pstride + i] = 0;
-  }
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o, 64);
-  if (lane != 0) return;
-  RsState s = st[i];
-  s.k++;
-  if (s.nan) {
-    s.done = RS_NAN;
-  } else if (c == 0) {
-    s.done = RS_SETTLED;
-  } else {
-    if (s.last >= 0 && (long long)c < s.last) s.falling = 1;
-    else if (s.last >= 0 && s.falling) s.settle = 1;
-    s.last = (long long)c;
-    if (s.k >= max_sweeps) s.done = RS_SWEEPS;
-  }
-  st[i] = s;
-  if (!s.done) atomicAdd(active, 1);
 }
 
 // the exclusive rank of a true predicate within the block (RS_B threads)
@@ -811,7 +851,7 @@ extern "C" int dcl_reinitialize_parallel(dcl_reinit_cell* cells, int ncells, int
     if (hipGetLastError() != hipSuccess) rc_ = set_error(DCL_ERR_LIB, "reinit reset / boundary launch failed");
   }
   // the sweeps, in groups of RS_GROUP: once a group is queued, the count of
-  // level sets still sweeping after the group before it is awaited (through
+  // level sets still sweeping late in the group before it is awaited (through
   // pinned memory), so the GPU always holds the next group; a level set
   // that has settled skips the sweeps queued after it
   static thread_local int* pin = nullptr;
@@ -827,32 +867,38 @@ extern "C" int dcl_reinitialize_parallel(dcl_reinit_cell* cells, int ncells, int
     hipError_t e = hipEventCreateWithFlags(&ev[q], hipEventDisableTiming);
     if (e != hipSuccess) rc_ = hip_fail(e, "reinit events", __FILE__, __LINE__);
   }
-  const unsigned ng = (unsigned)(nch < RS_NEED_GRID ? nch : RS_NEED_GRID);
+  const unsigned ng = (unsigned)(nch < RS_NEED_GRID ? nch : RS_NEED_GRID), nst = grid1d(ncells, RS_B / 64);
   bool settled = false;
   for (int j0 = 0, grp = 0; j0 < max_sweeps && !rc_ && !settled; j0 += RS_GROUP, ++grp) {
     const int j1 = j0 + RS_GROUP < max_sweeps ? j0 + RS_GROUP : max_sweeps;
     for (int j = j0; j < j1; ++j) {
-      hipLaunchKernelGGL(rs_need_k, dim3(ng), dim3(RS_B), 0, s, dcells, ncells, dstate, nch, nlist, ncount + j);
+      // with the state after sweep j - 1, into active[j - 1]
+      hipLaunchKernelGGL(rs_need_k, dim3(ng + (j > 0 ? nst : 0u)), dim3(RS_B), 0, s, dcells, ncells, dstate, nch, j,
+                         (int)ng, nlist, ncount + j, max_sweeps, active + (j > 0 ? j - 1 : 0), parts, nparts, pstride);
       if (d3)
         hipLaunchKernelGGL(rs_update_k<3>, dim3(RS_GRID), dim3(RS_B), 0, s, dcells, dstate, nlist, ncount + j, parts,
                            nparts, pstride);
       else
         hipLaunchKernelGGL(rs_update_k<2>, dim3(RS_GRID), dim3(RS_B), 0, s, dcells, dstate, nlist, ncount + j, parts,
                            nparts, pstride);
-      hipLaunchKernelGGL(rs_state_k, dim3(grid1d(ncells, RS_B / 64)), dim3(RS_B), 0, s, dstate, ncells, max_sweeps,
-                         active + j, parts, nparts, pstride);
     }
     if (hipGetLastError() != hipSuccess) {
       rc_ = set_error(DCL_ERR_LIB, "reinit sweep launch failed");
       break;
     }
-    hipError_t e = hipMemcpyAsync(pin + (grp & 1), active + (j1 - 1), sizeof(int), hipMemcpyDeviceToHost, s);
+    if (j1 < 2) continue;
+    hipError_t e = hipMemcpyAsync(pin + (grp & 1), active + (j1 - 2), sizeof(int), hipMemcpyDeviceToHost, s);
     if (e == hipSuccess) e = hipEventRecord(ev[grp & 1], s);
     if (e == hipSuccess && grp > 0) {
       e = hipEventSynchronize(ev[(grp - 1) & 1]);
       if (e == hipSuccess && pin[(grp - 1) & 1] == 0) settled = true;
     }
     if (e != hipSuccess) rc_ = hip_fail(e, "reinit sweeps", __FILE__, __LINE__);
+  }
+  if (!rc_ && !settled) {  // the last sweep's state
+    hipLaunchKernelGGL(rs_state_k, dim3(nst), dim3(RS_B), 0, s, dstate, ncells, max_sweeps, active + (max_sweeps - 1),
+                       parts, nparts, pstride);
+    if (hipGetLastError() != hipSuccess) rc_ = set_error(DCL_ERR_LIB, "reinit state launch failed");
   }
   for (int q = 0; q < 2; ++q)
     if (ev[q]) (void)hipEventDestroy(ev[q]);

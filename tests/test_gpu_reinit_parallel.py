@@ -160,6 +160,29 @@ def test_parallel_band_capacity_and_mixed_dims(dev):
         M.reinitialize_parallel([(to_dev(phi), win, drecs, len(recs)), (phi2, win2, empty, 0)])
 
 
+def test_parallel_every_node_marked(dev):
+    """Stripes of 6 nodes over a window of more than four chunks per block of
+    the mark scan: the boundary values mark every node at once, so a block
+    finds more marked nodes than it holds in LDS."""
+    nx, ny = 2002, 2201
+    win = D.GridWindow((-4, 9, 0), (nx, ny, 1), (1.0, 1.0, 1.0))
+    x = np.arange(nx)
+    k, d = x // 6, x % 6 - 0.3  # lines at 6 k + 0.3
+    dist = np.where(d < 3, d, d - 6)
+    phi = np.ascontiguousarray(np.broadcast_to(np.where(k % 2 == 0, 1.0, -1.0) * d, (ny, nx)))
+    at = np.flatnonzero((np.abs(dist) < 1))
+    recs = np.zeros((ny, len(at)), dtype=M.IRREGULAR_DTYPE)
+    recs["pos"][..., 0], recs["pos"][..., 1] = at[None, :] + win.p[0], np.arange(ny)[:, None] + win.p[1]
+    recs["axis"] = recs["shift"] = -1
+    recs["sign_center"] = np.where(phi[:, at] > 0, 1, -1)
+    recs["op"][..., 0] = -dist[at][None, :]
+    recs = np.ascontiguousarray(recs.reshape(-1))
+    drecs = torch.from_numpy(recs.view(np.uint8).reshape(-1)).to("cuda:0")
+    dphi = to_dev(phi)
+    (band,), (sweeps,) = M.reinitialize_parallel([(dphi, win, drecs, len(recs))])
+    _check(phi, win, recs, dphi, band, sweeps)
+
+
 def test_parallel_large_window_flat_path(dev):
     """A window of 2^28 nodes or more (700 x 700 x 600) takes the large-window
     path (64-bit pointer loads instead of 32-bit buffer offsets).  phi = 3 x
