@@ -40,29 +40,165 @@ __device__ __forceinline__ double dist2(double dx, double dy, double dz, bool th
 }
 
 // --------------------------------------------------------------- advect
-// BUF (3D, velocity window below 2 GiB): the MAC interpolations read with
-// buffer loads (32-bit offsets; with 3 FP32 components an x pair of faces is
-// one 16-byte load), the same arithmetic as the pointer path
-template <typename T, int DIM, bool BUF>
+// How the velocity is read: with pointers; with buffer loads (3D, velocity
+// window below 2 GiB: 32-bit offsets, and with 3 FP32 components an x pair of
+// faces is one 16-byte load); or, on top of these, from LDS boxes (exactly 3
+// components a node, a window no smaller than a box)
+enum { ADV_PTR, ADV_BUF, ADV_BOX };
+
+// The box of velocity nodes that a wave stages.  Particles lie in memory as
+// they were seeded, node by node along x, so the 64 of a wave sit around a few
+// neighbouring nodes of one row, and the 24 corner pairs that each interpolates
+// are nearly the same: gathered, they were 24 loads of 64 lanes per particle
+// against the 3 (FP64: 5) that bring the box.  8 nodes along x hold 4 cells
+// of particles, and 5 along y and z one cell, with the RK2 midpoint half a
+// cell away to either side; where a row of particles ends within a wave, the
+// rest of it has a second box, and lanes that neither box holds gather.
+// 8.8M FP32 particles in a band of the 256^3 window 227 -> 122 us: the texture
+// path was 94% busy, now the vector units are (82%; 420 instructions per
+// particle of which 84 are the six divisions by the spacing, against 52 us
+// for reading and writing the particles).
+constexpr int BOX_X = 8, BOX_Y = 5, BOX_Z = 5;
+constexpr int BOX_NODES = BOX_X * BOX_Y * BOX_Z;
+// Fewest particles that a wave stages a box for: a box costs the loads of a
+// quarter of one gathered interpolation.  Particles in no order would stage
+// boxes for a few lanes each and gather the others all the same.
+constexpr int BOX_MIN = 8;
+
+template <typename T>
+struct VelBox {
+  int o[3];  // the box's lowest node
+
+  __device__ __forceinline__ void place(const KVel& v, int x, int y, int z) {
+    o[0] = clampi(x - 1, 0, v.w.nx - BOX_X);
+    o[1] = clampi(y - 1, 0, v.w.ny - BOX_Y);
+    o[2] = clampi(z - 1, 0, v.w.nz - BOX_Z);
+  }
+  // whether all corners of the split (b0, b1) lie in the box (b0 <= b1 <= b0 + 1)
+  __device__ __forceinline__ bool holds(const int b0[3], const int b1[3]) const {
+    return (b0[0] >= o[0]) & (b1[0] <= o[0] + BOX_X - 2) & (b0[1] >= o[1]) & (b1[1] <= o[1] + BOX_Y - 2) &
+           (b0[2] >= o[2]) & (b1[2] <= o[2] + BOX_Z - 2);
+  }
+  // one 16-byte load per chunk of a row; rows lie in LDS as they do in memory
+  __device__ __forceinline__ void stage(rsrc_t rv, const KVel& v, T* lds, int lane) const {
+    constexpr int CH = 16 / (int)sizeof(T), RC = BOX_X * 3 / CH;  // elements of a chunk, chunks of a row
+    constexpr int NC = 3 * BOX_NODES / CH, PER = (NC + 63) / 64;
+    const int sy = v.w.nx * 3, sz = v.w.ny * sy, base = o[2] * sz + o[1] * sy + o[0] * 3;
+    T q[PER][CH];
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      const int c = min(lane + 64 * i, NC - 1), row = c / RC;
+      const int e = base + (row / BOX_Y) * sz + (row % BOX_Y) * sy + (c % RC) * CH;
+      if constexpr (CH == 4)
+        BL<T>::four(rv, e * (int)sizeof(T), 0, q[i]);
+      else
+        BL<T>::two(rv, e * (int)sizeof(T), 0, q[i]);
+    }
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      const int c = lane + 64 * i;
+      if (c >= NC) break;
+#pragma unroll
+      for (int k = 0; k < CH; ++k) lds[c * CH + k] = q[i][k];
+    }
+  }
+  // mac_vel_buf_split from the box at lds
+  __device__ __forceinline__ void vel(const T* lds, const int b0[3], const int b1[3], const T f0[3], const T f1[3],
+                                      T V[3]) const {
+    constexpr int sx = 3, sy = BOX_X * sx, sz = BOX_Y * sy;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      const int ix = c == 0 ? b1[0] : b0[0], iy = c == 1 ? b1[1] : b0[1], iz = c == 2 ? b1[2] : b0[2];
+      const T* b = lds + (iz - o[2]) * sz + (iy - o[1]) * sy + (ix - o[0]) * sx + c;
+      const T x1 = c == 0 ? f1[0] : f0[0], y1 = c == 1 ? f1[1] : f0[1], z1 = c == 2 ? f1[2] : f0[2];
+      V[c] = vtri(b[0], b[sx], b[sy], b[sy + sx], b[sz], b[sz + sx], b[sz + sy], b[sz + sy + sx], x1, y1, z1);
+    }
+  }
+};
+
+// both velocities of a particle's step (at X and at the midpoint) from the
+// boxes of its wave
+template <typename T>
+__device__ __forceinline__ void box_vels(rsrc_t rv, KVel v, const double X[3], double dt, const double dh[3],
+                                         T* lds, T V2[3]) {
+  v.dof = 3, v.udof = 0, v.cs = 1;
+  const int lane = threadIdx.x & 63;
+  int b0[3], b1[3];
+  T f0[3], f1[3], V1[3];
+  mac_split<T, 3>(v, X, b0, b1, f0, f1);
+  VelBox<T> A, B;
+  A.place(v, __builtin_amdgcn_readfirstlane(b0[0]), __builtin_amdgcn_readfirstlane(b0[1]),
+          __builtin_amdgcn_readfirstlane(b0[2]));
+  const bool inA = A.holds(b0, b1);
+  const unsigned long long ma = __builtin_amdgcn_ballot_w64(inA);
+  const bool useA = __popcll(ma) >= BOX_MIN;
+  bool inB = false;
+  if (~ma) {
+    const int l = __ffsll(~ma) - 1;
+    B.place(v, __builtin_amdgcn_readlane(b0[0], l), __builtin_amdgcn_readlane(b0[1], l),
+            __builtin_amdgcn_readlane(b0[2], l));
+    inB = B.holds(b0, b1) && !inA;
+  } else {
+    B = A;
+  }
+  const bool useB = __popcll(__builtin_amdgcn_ballot_w64(inB)) >= BOX_MIN;
+  if (useA) A.stage(rv, v, lds, lane);
+  if (useB) B.stage(rv, v, lds + 3 * BOX_NODES, lane);
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  const bool second = inB && useB, boxed = second || (inA && useA);
+  const T* box = second ? lds + 3 * BOX_NODES : lds;
+  VelBox<T> own;
+#pragma unroll
+  for (int a = 0; a < 3; ++a) own.o[a] = second ? B.o[a] : A.o[a];
+  if (boxed)
+    own.vel(box, b0, b1, f0, f1, V1);
+  else
+    mac_vel_buf_split<T>(rv, v, b0, b1, f0, f1, V1);
+  double Xm[3];
+#pragma unroll
+  for (int a = 0; a < 3; ++a) Xm[a] = X[a] + dt / 2 * (double)V1[a] / dh[a];
+  mac_split<T, 3>(v, Xm, b0, b1, f0, f1);
+  if (boxed && own.holds(b0, b1))
+    own.vel(box, b0, b1, f0, f1, V2);
+  else
+    mac_vel_buf_split<T>(rv, v, b0, b1, f0, f1, V2);
+}
+
+template <typename T, int DIM, int MODE>
 __global__ __launch_bounds__(256) void pls_advect_k(T* __restrict__ P, int64_t n,
                                                     const T* __restrict__ vel, KVel v,
                                                     double dhx, double dhy, double dhz, double dt,
                                                     unsigned vbytes) {
   const int64_t m = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const double dh[3] = {dhx, dhy, dhz};
+  if constexpr (MODE == ADV_BOX) {
+    __shared__ __attribute__((aligned(16))) T boxes[256 / 64][2][3 * BOX_NODES];
+    // the wave's lanes past the end go along with its last particle
+    if (m - (threadIdx.x & 63) >= n) return;
+    T* p = P + 4 * (m < n ? m : n - 1);
+    const double X[3] = {(double)p[0], (double)p[1], (double)p[2]};
+    T V2[3];
+    box_vels<T>(make_rsrc(vel, vbytes), v, X, dt, dh, boxes[threadIdx.x / 64][0], V2);
+    if (m >= n) return;
+#pragma unroll
+    for (int a = 0; a < 3; ++a) p[a] = (T)(X[a] + dt * (double)V2[a] / dh[a]);
+    return;
+  }
   if (m >= n) return;
   T* p = P + 4 * m;
-  const double dh[3] = {dhx, dhy, dhz};
   double X[3] = {(double)p[0], (double)p[1], (double)p[2]};
   T V1[3], V2[3];
   const rsrc_t rv = make_rsrc(vel, vbytes);
-  if (BUF && DIM == 3)
+  if (MODE == ADV_BUF)
     mac_vel_buf<T>(rv, v, X, V1);
   else
     mac_vel<T, DIM>(vel, v, X, V1);
   double Xm[3] = {X[0], X[1], X[2]};
 #pragma unroll
   for (int a = 0; a < DIM; ++a) Xm[a] = X[a] + dt / 2 * (double)V1[a] / dh[a];
-  if (BUF && DIM == 3)
+  if (MODE == ADV_BUF)
     mac_vel_buf<T>(rv, v, Xm, V2);
   else
     mac_vel<T, DIM>(vel, v, Xm, V2);
@@ -269,19 +405,22 @@ extern "C" int dcl_pls_advect(void* particles, int64_t count, const dcl_velocity
   hipStream_t s = as_stream(stream);
   const unsigned g = grid1d(count, 256);
   const long long vb = win_nodes(vel->win) * vel->dof * (long long)(precision == DCL_F64 ? 8 : 4);
-  const bool buf = dim == 3 && buf_ok(0, vb);
-#define DCL_ADV(T, D)                                                                                     \
-  if (buf)                                                                                              \
-    hipLaunchKernelGGL((pls_advect_k<T, D, true>), dim3(g), dim3(256), 0, s, static_cast<T*>(particles),  \
-                       count, static_cast<const T*>(vel->data), v, dh.x, dh.y, dh.z, dt, (unsigned)vb);   \
-  else                                                                                                  \
-    hipLaunchKernelGGL((pls_advect_k<T, D, false>), dim3(g), dim3(256), 0, s, static_cast<T*>(particles), \
-                       count, static_cast<const T*>(vel->data), v, dh.x, dh.y, dh.z, dt, 0u)
+  int mode = dim == 3 && buf_ok(0, vb) ? ADV_BUF : ADV_PTR;
+  if (mode == ADV_BUF && v.dof == 3 && v.w.nx >= BOX_X && v.w.ny >= BOX_Y && v.w.nz >= BOX_Z) mode = ADV_BOX;
+#define DCL_ADV(T, D, M)                                                                             \
+  hipLaunchKernelGGL((pls_advect_k<T, D, M>), dim3(g), dim3(256), 0, s, static_cast<T*>(particles),  \
+                     count, static_cast<const T*>(vel->data), v, dh.x, dh.y, dh.z, dt, (unsigned)vb)
+#define DCL_ADV_T(T)                             \
+  if (dim == 2) DCL_ADV(T, 2, ADV_PTR);          \
+  else if (mode == ADV_PTR) DCL_ADV(T, 3, ADV_PTR);   \
+  else if (mode == ADV_BUF) DCL_ADV(T, 3, ADV_BUF);   \
+  else DCL_ADV(T, 3, ADV_BOX)
   if (precision == DCL_F64) {
-    if (dim == 3) DCL_ADV(double, 3); else DCL_ADV(double, 2);
+    DCL_ADV_T(double);
   } else {
-    if (dim == 3) DCL_ADV(float, 3); else DCL_ADV(float, 2);
+    DCL_ADV_T(float);
   }
+#undef DCL_ADV_T
 #undef DCL_ADV
   DCL_LAUNCHED("pls_advect");
   return 0;

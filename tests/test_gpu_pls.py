@@ -51,6 +51,43 @@ def test_advect_particles(dev, dtype, tol, dim):
     assert np.array_equal(got[:, 3], ref[:, 3])
 
 
+# FP32: V1 to 2e-7 moves the midpoint by up to 2 cells * 2e-7 = 4e-7 of a cell,
+# there V2 changes by up to 2 per cell: 1e-6 with its own rounding, times 4
+# cells, plus the rounding of a position of up to 16 or 32: 5e-6 cells of 8
+@pytest.mark.parametrize("dtype,tol", [(torch.float64, 1e-12), (torch.float32, 2e-6)])
+@pytest.mark.parametrize("n,dof,order", [((8, 5, 5), 3, "rows"), ((7, 5, 5), 3, "rows"), ((24, 5, 9), 3, "rows"),
+                                         ((31, 17, 13), 3, "rows"), ((31, 17, 13), 4, "rows"),
+                                         ((31, 17, 13), 3, "mixed"), ((31, 17, 13), 3, "random")])
+@pytest.mark.parametrize("cells", [0.3, 4.0])
+def test_advect_particles_velocity_boxes(dev, dtype, tol, n, dof, order, cells):
+    """Particles around every node, row by row (two boxes where a row ends
+    within a wave), partly or wholly out of order (waves that gather), moved
+    within their box and out of it, some outside the window, and an end of
+    the list within a wave."""
+    rng = np.random.default_rng(7)
+    win = D.GridWindow((3, -2, 5), n, (0.5, 0.5, 0.5))
+    vel = rng.uniform(-1.0, 1.0, (n[2], n[1], n[0], dof))
+    nodes = np.stack(np.meshgrid(*(np.arange(k) for k in n[::-1]), indexing="ij"), -1).reshape(-1, 3)[:, ::-1]
+    P = np.zeros((11 * len(nodes), 4))
+    P[:, :3] = np.repeat(nodes, 11, 0) + rng.uniform(-0.5, 0.5, (len(P), 3)) + np.array(win.p)
+    P[:, 3] = rng.uniform(-0.5, 0.5, len(P))
+    P[::97, :3] += rng.uniform(-9.0, 9.0, P[::97, :3].shape)
+    if order == "mixed":
+        k = rng.choice(len(P), len(P) // 3, replace=False)
+        P[np.sort(k)] = P[k]
+    if order == "random":
+        P = P[rng.permutation(len(P))]
+    P = P[:len(P) - len(P) % 64 + 37]
+    P, vel = rounded(P, dtype), rounded(vel, dtype)
+    dt = cells * win.d[0]
+    Pd = to_dev(P, dtype)
+    PL.advect_particles(Pd, to_dev(vel, dtype), win, win.d, dt)
+    ref = O.pls_advect(P, vel, owin(win), win.d, dt, 3)
+    got = to_np(Pd)
+    assert rel_max(got[:, :3], ref[:, :3], float(max(n))) <= tol
+    assert np.array_equal(got[:, 3], ref[:, 3])
+
+
 def _interp(phi, win, P, dim):
     """Plain (bi/tri)linear phi at particle positions (numpy)."""
     pos = P[:, :3] - np.array(win.p, dtype=np.float64)
