@@ -40,6 +40,32 @@ int device_cus();
 // their stream before returning, so the buffer is free again on return.
 int scratch(size_t bytes, void** ptr);
 
+// A few words of pinned host memory for the result of a synchronous entry
+// point: its last kernel writes them there and wait() synchronises the
+// stream.  A kernel and its result come back in 13.9 us that way, against
+// 22.6 us with a copy to the caller's pageable word, which is staged and
+// awaited by itself.  The words are one of HR_SLOTS of the process, allocated
+// together by the first call that needs one (all in use: an allocation of the
+// call's own); they are given back once the stream has been waited for, and
+// stay taken where that failed, since a kernel may still write them.
+class HostResult {
+ public:
+  static constexpr int HR_SLOTS = 64, HR_BYTES = 64;
+  HostResult() = default;
+  ~HostResult();
+  HostResult(const HostResult&) = delete;
+  HostResult& operator=(const HostResult&) = delete;
+  int take();
+  int wait(hipStream_t s);
+  template <typename V>
+  V* as() const { return static_cast<V*>(p_); }
+
+ private:
+  void* p_ = nullptr;
+  int slot_ = -1;
+  bool waited_ = false;
+};
+
 // Exclusive scan of per-block counts (scan.hip), in two levels over tiles of
 // SCAN_TILE counts: afterwards the exclusive prefix of count i is
 // counts[i] + sums[i / SCAN_TILE] and *total is the sum.  A tile's prefix must

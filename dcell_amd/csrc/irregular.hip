@@ -721,29 +721,28 @@ static int irregular_t(const void* phi, const dcl_window* win, const dcl_icoor* 
                        dcl_irregular_node* out, int64_t cap, int64_t* count_out, hipStream_t s) {
   const int64_t nblk = (nb + IRB - 1) / IRB;
   const int64_t ntiles = scan_tiles(nblk);
-  // scratch: 2 totals | 2 x tile sums | 2 x block counts (16-byte padded) | tasks (one per band node at most)
+  // scratch: projection total | 2 x tile sums | 2 x block counts (16-byte padded) | tasks (one per band node at most)
   const size_t counts_bytes = ((sizeof(unsigned) * nblk + 15) / 16) * 16;
   const size_t sums_off = 16, counts_off = sums_off + 2 * sizeof(unsigned long long) * ntiles;
   const size_t tasks_off = ((counts_off + 2 * counts_bytes + 15) / 16) * 16;
   void* sc = nullptr;
   DCL_TRY(scratch(tasks_off + sizeof(IrrTask) * (size_t)nb, &sc));
   char* base = static_cast<char*>(sc);
-  unsigned long long* totals = reinterpret_cast<unsigned long long*>(base);
+  HostResult records;
+  DCL_TRY(records.take());
   unsigned long long* sums = reinterpret_cast<unsigned long long*>(base + sums_off);
   unsigned* counts = reinterpret_cast<unsigned*>(base + counts_off);
   const ScanArrays sa = {{counts, reinterpret_cast<unsigned*>(base + counts_off + counts_bytes)},
                          {sums, sums + ntiles},
-                         {totals, totals + 1}};
+                         {records.as<unsigned long long>(), reinterpret_cast<unsigned long long*>(base)}};
   IrrTask* tasks = reinterpret_cast<IrrTask*>(base + tasks_off);
   const T* p = static_cast<const T*>(phi);
   const KWin w = kwin(*win);
   const int rc = win->n.z >= 2 ? irr_launch<T, 3>(p, w, band, nb, sa, tasks, out, cap, s)
                                : irr_launch<T, 2>(p, w, band, nb, sa, tasks, out, cap, s);
   if (rc) return rc;
-  unsigned long long tot = 0;
-  DCL_HIP(hipMemcpyAsync(&tot, totals, sizeof(tot), hipMemcpyDeviceToHost, s));
-  DCL_HIP(hipStreamSynchronize(s));
-  *count_out = (int64_t)tot;
+  DCL_TRY(records.wait(s));
+  *count_out = (int64_t)*records.as<unsigned long long>();
   return 0;
 }
 

@@ -191,12 +191,6 @@ __global__ __launch_bounds__(RB) void norms_k(const TA* __restrict__ a, const TB
   block_reduce<3>(v, kind, part + 3 * blockIdx.x);
 }
 
-static int fetch(double* host, const double* dev, int count, hipStream_t s) {
-  DCL_HIP(hipMemcpyAsync(host, dev, sizeof(double) * count, hipMemcpyDeviceToHost, s));
-  DCL_HIP(hipStreamSynchronize(s));
-  return 0;
-}
-
 }  // namespace dcl
 
 using namespace dcl;
@@ -218,8 +212,10 @@ extern "C" int dcl_max_velocity(const dcl_velocity* vel, const void* nodes, int6
   const KVel v = kvel(*vel);
   const int nb = (int)(grid1d(count, RB) < (unsigned)RGRID ? grid1d(count, RB) : RGRID);
   void* sc = nullptr;
-  DCL_TRY(scratch(sizeof(double) * (nb + 1), &sc));
+  DCL_TRY(scratch(sizeof(double) * nb, &sc));
   double* part = static_cast<double*>(sc);
+  HostResult res;
+  DCL_TRY(res.take());
   hipStream_t s = as_stream(stream);
   const char* nd = static_cast<const char*>(nodes);
 #define DCL_MV(T, D)                                                                        \
@@ -232,15 +228,17 @@ extern "C" int dcl_max_velocity(const dcl_velocity* vel, const void* nodes, int6
   }
 #undef DCL_MV
   DCL_LAUNCHED("maxvel");
-  hipLaunchKernelGGL((fold_partials_k<1>), dim3(1), dim3(RB), 0, s, part, nb, part + nb, 1, 0, 0, 0);
+  hipLaunchKernelGGL((fold_partials_k<1>), dim3(1), dim3(RB), 0, s, part, nb, res.as<double>(), 1, 0, 0, 0);
   DCL_LAUNCHED("fold_partials");
-  return fetch(max_out, part + nb, 1, s);
+  DCL_TRY(res.wait(s));
+  *max_out = res.as<double>()[0];
+  return 0;
 }
 
-// scratch of a band compaction: total | tile sums | block counts
+// scratch of a band compaction: tile sums | block counts
 static size_t band_scratch_bytes(int64_t n) {
   const int64_t nb = grid1d(n, RB);
-  return 16 + sizeof(unsigned long long) * scan_tiles(nb) + sizeof(unsigned) * nb;
+  return sizeof(unsigned long long) * scan_tiles(nb) + sizeof(unsigned) * nb;
 }
 
 // The allocation-free band compaction's scratch: one array per device, held
@@ -275,23 +273,22 @@ static int band_compact_t(const void* phi, const dcl_window* win, double width, 
   const int64_t n = win_nodes(*win);
   const int64_t nb = grid1d(n, RB);
   const int64_t ntiles = scan_tiles(nb);
-  unsigned long long* total = static_cast<unsigned long long*>(sc);
-  unsigned long long* sums = total + 2;
+  HostResult total;
+  DCL_TRY(total.take());
+  unsigned long long* sums = static_cast<unsigned long long*>(sc);
   unsigned* counts = reinterpret_cast<unsigned*>(sums + ntiles);
   const T* p = static_cast<const T*>(phi);
   hipLaunchKernelGGL((band_count_k<T>), dim3(nb), dim3(RB), 0, s, p, n, (T)width, counts);
   DCL_LAUNCHED("band_count");
-  const ScanArrays sa = {{counts, nullptr}, {sums, nullptr}, {total, nullptr}};
+  const ScanArrays sa = {{counts, nullptr}, {sums, nullptr}, {total.as<unsigned long long>(), nullptr}};
   DCL_TRY(scan_counts(sa, 1, nb, s));
   if (cap > 0) {
     hipLaunchKernelGGL((band_write_k<T>), dim3(nb), dim3(RB), 0, s, p, kwin(*win), n, (T)width, counts, sums,
                        out, cap);
     DCL_LAUNCHED("band_write");
   }
-  unsigned long long tot = 0;
-  DCL_HIP(hipMemcpyAsync(&tot, total, sizeof(tot), hipMemcpyDeviceToHost, s));
-  DCL_HIP(hipStreamSynchronize(s));
-  *count_out = (int64_t)tot;
+  DCL_TRY(total.wait(s));
+  *count_out = (int64_t)*total.as<unsigned long long>();
   return 0;
 }
 
@@ -343,8 +340,10 @@ extern "C" int dcl_interface_metrics(const void* phi, const void* kappa, const d
   const int dim = win->n.z < 2 ? 2 : 3;
   const int nb = RGRID;
   void* sc = nullptr;
-  DCL_TRY(scratch(sizeof(double) * 3 * (nb + 1), &sc));
+  DCL_TRY(scratch(sizeof(double) * 3 * nb, &sc));
   double* part = static_cast<double*>(sc);
+  HostResult res;
+  DCL_TRY(res.take());
   hipStream_t s = as_stream(stream);
   const KWin w = kwin(*win);
 #define DCL_MT(T, D)                                                                             \
@@ -357,10 +356,10 @@ extern "C" int dcl_interface_metrics(const void* phi, const void* kappa, const d
   }
 #undef DCL_MT
   DCL_LAUNCHED("interface_metrics");
-  hipLaunchKernelGGL((fold_partials_k<3>), dim3(1), dim3(RB), 0, s, part, nb, part + 3 * nb, 0, 0, 0, 0);
+  hipLaunchKernelGGL((fold_partials_k<3>), dim3(1), dim3(RB), 0, s, part, nb, res.as<double>(), 0, 0, 0, 0);
   DCL_LAUNCHED("fold_partials");
-  double r[3];
-  DCL_TRY(fetch(r, part + 3 * nb, 3, s));
+  DCL_TRY(res.wait(s));
+  const double* r = res.as<double>();
   out[0] = r[0];
   out[1] = r[1];
   out[2] = r[0] > 0 ? r[1] / r[0] : 0.0;
@@ -380,8 +379,10 @@ extern "C" int dcl_error_norms(const void* a, int prec_a, const void* b, int pre
   if (n == 0) return 0;
   const int nb = (int)(grid1d(n, RB) < (unsigned)RGRID ? grid1d(n, RB) : RGRID);
   void* sc = nullptr;
-  DCL_TRY(scratch(sizeof(double) * 3 * (nb + 1), &sc));
+  DCL_TRY(scratch(sizeof(double) * 3 * nb, &sc));
   double* part = static_cast<double*>(sc);
+  HostResult res;
+  DCL_TRY(res.take());
   hipStream_t s = as_stream(stream);
 #define DCL_NM(TA, TB)                                                                         \
   hipLaunchKernelGGL((norms_k<TA, TB>), dim3(nb), dim3(RB), 0, s, static_cast<const TA*>(a),       \
@@ -392,7 +393,9 @@ extern "C" int dcl_error_norms(const void* a, int prec_a, const void* b, int pre
   else DCL_NM(float, float);
 #undef DCL_NM
   DCL_LAUNCHED("error_norms");
-  hipLaunchKernelGGL((fold_partials_k<3>), dim3(1), dim3(RB), 0, s, part, nb, part + 3 * nb, 1, 0, 1, 0);
+  hipLaunchKernelGGL((fold_partials_k<3>), dim3(1), dim3(RB), 0, s, part, nb, res.as<double>(), 1, 0, 1, 0);
   DCL_LAUNCHED("fold_partials");
-  return fetch(out, part + 3 * nb, 3, s);
+  DCL_TRY(res.wait(s));
+  for (int k = 0; k < 3; ++k) out[k] = res.as<double>()[k];
+  return 0;
 }

@@ -1,6 +1,7 @@
 // runtime.hip -- error reporting, argument checks and the memory helpers of
 // the C ABI (dcell_lsm.h).
 #include <atomic>
+#include <mutex>
 #include <stdio.h>
 #include <string.h>
 
@@ -98,6 +99,46 @@ int scratch(size_t bytes, void** ptr) {
   }
   *ptr = s.ptr;
   return 0;
+}
+
+static std::mutex g_hr_mu;
+static char* g_hr;
+static uint64_t g_hr_used;  // one bit a slot
+
+int HostResult::take() {
+  static_assert(HR_SLOTS == 64, "one bit of g_hr_used a slot");
+  {
+    std::lock_guard<std::mutex> lock(g_hr_mu);
+    if (!g_hr) {
+      void* p = nullptr;
+      DCL_HIP(hipHostMalloc(&p, HR_SLOTS * HR_BYTES, hipHostMallocPortable));
+      g_hr = static_cast<char*>(p);
+    }
+    if (~g_hr_used) {
+      slot_ = __builtin_ctzll(~g_hr_used);
+      g_hr_used |= (uint64_t)1 << slot_;
+      p_ = g_hr + slot_ * HR_BYTES;
+      return 0;
+    }
+  }
+  DCL_HIP(hipHostMalloc(&p_, HR_BYTES, hipHostMallocPortable));
+  return 0;
+}
+
+int HostResult::wait(hipStream_t s) {
+  DCL_HIP(hipStreamSynchronize(s));
+  waited_ = true;
+  return 0;
+}
+
+HostResult::~HostResult() {
+  if (!p_ || !waited_) return;
+  if (slot_ < 0) {
+    (void)hipHostFree(p_);
+    return;
+  }
+  std::lock_guard<std::mutex> lock(g_hr_mu);
+  g_hr_used &= ~((uint64_t)1 << slot_);
 }
 
 // Streaming device copy: 16-byte elements, each thread keeps SC_U loads in

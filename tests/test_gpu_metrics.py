@@ -1,6 +1,7 @@
 """Parity of the gfx950 reductions (max velocity, band compaction, interface
 metrics, error norms) with the oracle."""
 import math
+import threading
 
 import numpy as np
 import pytest
@@ -32,6 +33,38 @@ def test_max_velocity_with_irregular_node_stride(dev, dim):
     assert got == pytest.approx(ref, rel=1e-15)
     got32 = M.max_velocity(to_dev(vel, torch.float32), win, to_dev(nodes, torch.int32))
     assert got32 == pytest.approx(ref, rel=1e-6)
+
+
+@pytest.mark.parametrize("threads", [3, 80])
+def test_host_results_of_concurrent_calls(dev, threads):
+    """Each thread's calls return its own result, also with more calls under
+    way than the process keeps host words for."""
+    n = 24
+    win = D.GridWindow((0, 0, 0), (n, n, n), (1.0, 1.0, 1.0))
+    vel = random_velocity(n, 3, np.random.default_rng(3), 1.0)
+    phi = smooth_field(n, 3, np.random.default_rng(4))
+    dvel, dphi = to_dev(vel), to_dev(phi)
+    nodes = [np.array([[1 + i % 20, 2 + i // 20, 3]], dtype=np.int32) for i in range(threads)]
+    widths = [0.02 * np.abs(phi).max() * (1 + i % 7) for i in range(threads)]
+    dnodes = [torch.from_numpy(q).to("cuda:0") for q in nodes]
+    torch.cuda.synchronize()
+    got, start = [None] * threads, threading.Barrier(threads)
+
+    def work(i):
+        with torch.cuda.stream(torch.cuda.Stream()):
+            start.wait()
+            got[i] = [(M.max_velocity(dvel, win, dnodes[i]), int(M.band_compact(dphi, win, widths[i])[1]))
+                      for _ in range(4)]
+
+    ts = [threading.Thread(target=work, args=(i,)) for i in range(threads)]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    for i in range(threads):
+        ref = O.max_velocity(vel, owin(win), nodes[i]), int((np.abs(phi) < widths[i]).sum())
+        for v, count in got[i]:
+            assert abs(v - ref[0]) <= 1e-14 * ref[0] and count == ref[1]
 
 
 @pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
