@@ -137,10 +137,24 @@ __device__ __forceinline__ void rs_mark(const RsCell& c, unsigned char* nd_, uns
   }
 }
 
+// what the first sweep finds: per level set its state, per sweep the counts
+// of active level sets and listed nodes, and the partial counts of a sweep
+struct RsStart {
+  RsState* state;
+  int *active, *ncount;
+  unsigned long long* parts;
+  int ncells, sweeps, nparts;
+};
+
 // FMM_InitializeEikonal (FastMarching.c:46-58): phi to +-PHI_INF in both
-// buffers; the mask keeps each node's side
-__global__ __launch_bounds__(RS_B) void rs_reset_k(const RsCell* __restrict__ cells, int ncells, long long nq) {
-  const long long g = blockIdx.x;
+// buffers; the mask keeps each node's side.  The grid sets z up too: three
+// fills and an upload before it took 20 us of a call.
+__global__ __launch_bounds__(RS_B) void rs_reset_k(const RsCell* __restrict__ cells, int ncells, long long nq,
+                                                   RsStart z) {
+  const long long g = blockIdx.x, all = (long long)gridDim.x * RS_B;
+  for (long long e = g * RS_B + threadIdx.x; e < z.ncells; e += all) z.state[e] = {0, 0, 0, 0, -1, 0, 0};
+  for (long long e = g * RS_B + threadIdx.x; e < z.sweeps; e += all) z.active[e] = z.ncount[e] = 0;
+  for (long long e = g * RS_B + threadIdx.x; e < z.nparts; e += all) z.parts[e] = 0;
   if (g >= nq) return;
   const RsCell& c = cells[rs_find<RS_KEY_RASTER>(cells, ncells, g)];
   const int64_t i = (g - c.qb0) * RS_B + threadIdx.x;
@@ -829,21 +843,15 @@ extern "C" int dcl_reinitialize_parallel(dcl_reinit_cell* cells, int ncells, int
     c.count = u.count;
     c.band = u.band;
     c.band_cap = u.band_capacity;
-    RsState& q = hstate[i];
-    memset(&q, 0, sizeof(q));
-    q.last = -1;
   }
   int rc_ = 0;
   {
     hipError_t e = hipMemcpyAsync(dcells, host, sizeof(RsCell) * ncells, hipMemcpyHostToDevice, s);
-    if (e == hipSuccess) e = hipMemcpyAsync(dstate, hstate, sizeof(RsState) * ncells, hipMemcpyHostToDevice, s);
-    if (e == hipSuccess) e = hipMemsetAsync(active, 0, sizeof(int) * (size_t)(max_sweeps + 1), s);
-    if (e == hipSuccess) e = hipMemsetAsync(ncount, 0, sizeof(int) * (size_t)(max_sweeps + 1), s);
-    if (e == hipSuccess) e = hipMemsetAsync(parts, 0, sizeof(unsigned long long) * (size_t)nparts * pstride, s);
     if (e != hipSuccess) rc_ = hip_fail(e, "reinit upload", __FILE__, __LINE__);
   }
   if (!rc_) {
-    hipLaunchKernelGGL(rs_reset_k, dim3((unsigned)nq), dim3(RS_B), 0, s, dcells, ncells, nq);
+    hipLaunchKernelGGL(rs_reset_k, dim3((unsigned)nq), dim3(RS_B), 0, s, dcells, ncells, nq,
+                       RsStart{dstate, active, ncount, parts, ncells, max_sweeps + 1, nparts * pstride});
     if (nr > 0) {
       if (d3) hipLaunchKernelGGL(rs_bc_k<3>, dim3((unsigned)nr), dim3(RS_B), 0, s, dcells, ncells, nr);
       else hipLaunchKernelGGL(rs_bc_k<2>, dim3((unsigned)nr), dim3(RS_B), 0, s, dcells, ncells, nr);
