@@ -295,10 +295,22 @@ __device__ __forceinline__ void ring_put(T* p, T v) {
 // ring (RG_R * G::PP values).
 template <typename T, int INTERP, int BT, typename G, int VM>
 __device__ __forceinline__ void ring_column(const T* __restrict__ phi0, T* __restrict__ phi, rsrc_t rp,
-                                            rsrc_t rv, const SLP& P, int x0, int y0, int z0, int zc, T* ring,
+                                            rsrc_t rv, const SLP& Pin, int x0, int y0, int z0, int zc, T* ring,
                                             T* vr) {
   typedef VelGeom<G::TX, G::TY, G::VRP, G::VPP> V;
   constexpr bool VL = VM == RV_STAGED, planes = VM == RV_PLANES;
+  SLP P = Pin;
+  // The staged velocity's window is phi's, 3 components a node: said here,
+  // the two windows share their scalar registers (of 31 spills into vector
+  // lanes 12 are left), the midpoint's fallback keeps one layout, and the
+  // kernel takes 71 vector registers instead of 104 (FP32 384^3 tricubic RK2
+  // step with its curvature 751 -> 732 us, 200^3 trilinear 147 -> 141 us)
+  if constexpr (VL) {
+    P.v.w = P.w;
+    P.v.dof = 3;
+    P.v.udof = 0;
+    P.v.cs = 1;
+  }
   const int nx = P.w.nx, ny = P.w.ny, nz = P.w.nz;
   const int z1 = min(nz, z0 + zc);
   const int tid = threadIdx.x + G::TX * threadIdx.y;
@@ -339,7 +351,8 @@ __device__ __forceinline__ void ring_column(const T* __restrict__ phi0, T* __res
     for (int q = 0; q < 4; ++q) mc.hi[c][q] = T(0);
   }
   NodeFaces<T> nf = {T(0), T(0), T(0), T(0), T(0)};
-  for (int k = z0; k < z1; ++k) {
+  int vb = 0;  // velocity ring slot of plane k - 1, (k - z0) mod VR_R
+  for (int k = z0; k < z1; ++k, vb = vb == VR_R - 1 ? 0 : vb + 1) {
     const int zn = k + RG_H + 1;
     const bool pre = zn < nz && k + 1 < z1;
     T pf[G::PF];
@@ -354,8 +367,9 @@ __device__ __forceinline__ void ring_column(const T* __restrict__ phi0, T* __res
       } else {
         double S[3];
         if constexpr (VL) {
-          const int b = (k - z0) % VR_R;
-          const int sl[4] = {b, (b + 1) % VR_R, (b + 2) % VR_R, (b + 3) % VR_R};
+          int sl[4];
+#pragma unroll
+          for (int m = 0; m < 4; ++m) sl[m] = vb + m < VR_R ? vb + m : vb + m - VR_R;
           sl_dep3_ring<T, BT, V>(rv, vr, sl, P, i, j, k, x0, y0, S);
         } else if constexpr (planes) {
           const int vz0 = P.v.w.pz, vz1 = P.v.w.pz + P.v.w.nz - 2;
@@ -399,15 +413,16 @@ __device__ __forceinline__ void ring_column(const T* __restrict__ phi0, T* __res
       }
     }
     if (pre) ring_store<T, G>(ring, (zn - z0 + RG_H) & (RG_R - 1), tid, so, pf);
-    if (vpre) vring_store<T, V>(vr, (k + 3 - z0 + 1) % VR_R, tid, vso, vf);
+    if (vpre) vring_store<T, V>(vr, vb == 0 ? VR_R - 1 : vb - 1, tid, vso, vf);  // (k + 3 - z0 + 1) mod VR_R
     __syncthreads();
   }
 }
 
 // Waves per SIMD the ring kernels are compiled for: the FP32 velocity-ring
 // kernel's LDS (40 KB per 256-thread block) admits 4 blocks per CU, and
-// asking for 4 waves per SIMD brings its registers from 136 to 104 (no
-// spills), 7% faster at 384^3; the others keep the compiler's choice.
+// its registers are held to those 4 waves per SIMD (left to the compiler
+// they were 136 where 104 do, 7% slower at 384^3); the others keep the
+// compiler's choice.
 template <typename T, int VM>
 constexpr int ring_waves() {
   return sizeof(T) == 4 && VM == RV_STAGED ? 4 : 1;
