@@ -37,6 +37,7 @@ struct BCell {
   int pad;
   double c[3], ch[3];  // dt / dh, dt / (2 dh)
   double dx, dy, dz;
+  double r2[5];        // 2D: curv2d_recips in the batch's precision
 };
 
 struct TileShape {
@@ -222,8 +223,11 @@ __global__ __launch_bounds__(Step2<T2R>::NT) void batch2d_step_k(const T* __rest
   claim_tiles(q, bounds, k, [&](int t) {
     const int4 tl = tiles[t];
     const BCell c = cells[tl.x];
+    Curv2R<T> cr;
+#pragma unroll
+    for (int q = 0; q < 5; ++q) cr.r[q] = (T)c.r2[q];
     step2d_tile<T, INTERP, BT, T2R>(phi0 + c.phi_off, phi + c.phi_off, kappa + c.phi_off, vel + c.vel_off,
-                                    cell_slp<2>(c), curv_recips<T>(c.dx, c.dy, 1.0), tl.y, tl.z, S);
+                                    cell_slp<2>(c), (T)c.dx, (T)c.dy, cr, tl.y, tl.z, S);
   });
 }
 
@@ -562,6 +566,11 @@ extern "C" int dcl_batch_create(int32_t ncells, const dcl_window* wins, int prec
     cell.px = w.p.x; cell.py = w.p.y; cell.pz = w.p.z;
     cell.nx = w.n.x; cell.ny = w.n.y; cell.nz = dim == 2 ? 1 : w.n.z;
     cell.dx = w.d.x; cell.dy = w.d.y; cell.dz = w.d.z;
+    if (dim == 2) {
+      const Curv2R<double> r = curv2d_recips<double>(w.d.x, w.d.y);
+      const Curv2R<float> rf = curv2d_recips<float>((float)w.d.x, (float)w.d.y);
+      for (int q = 0; q < 5; ++q) cell.r2[q] = precision == DCL_F64 ? r.r[q] : (double)rf.r[q];
+    }
     b->phi_off.push_back(po);
     b->vel_off.push_back(vo);
     b->host_cells.push_back(cell);

@@ -238,21 +238,28 @@ __device__ __forceinline__ T trilinear(const T* __restrict__ phi, const KWin& w,
                            (T)(1.0 - fy), (T)(1.0 - fz));
 }
 
-// Bilinear2D (Common/Grid.c:190-212): the (2x-1) form, x outer, y inner, /4
+// Bilinear2D (Common/Grid.c:190-212) from the rows y and y + 1: the (2x-1)
+// form, x outer, y inner, / 4, with every product-sum contracted
+template <typename T>
+__device__ __forceinline__ T bilinear_sum2d(const T r0[2], const T r1[2], double fx, double fy) {
+#pragma clang fp contract(off)
+  const T xf = (T)(2. * fx - 1.), yf = (T)(2. * fy - 1.);
+  const T xb0 = T(1) - xf, xb1 = T(1) + xf, yb0 = T(1) - yf, yb1 = T(1) + yf;
+  T sum = (r0[0] * xb0) * yb0;
+  sum = fma(r1[0] * xb0, yb1, sum);
+  sum = fma(r0[1] * xb1, yb0, sum);
+  sum = fma(r1[1] * xb1, yb1, sum);
+  return sum / T(4);
+}
+
 template <typename T>
 __device__ __forceinline__ T bilinear_ref2d(const T* __restrict__ phi, const KWin& w, const double S[2]) {
   double fx, fy;
   const int xi = lin_split(S[0], w.px, w.nx, fx);
   const int yi = lin_split(S[1], w.py, w.ny, fy);
-  const T xf = (T)(2. * fx - 1.), yf = (T)(2. * fy - 1.);
-  const T xb0 = T(1) - xf, xb1 = T(1) + xf, yb0 = T(1) - yf, yb1 = T(1) + yf;
   const T* b = phi + yi * w.nx + xi;
-  T sum = T(0);
-  sum += b[0] * xb0 * yb0;
-  sum += b[w.nx] * xb0 * yb1;
-  sum += b[1] * xb1 * yb0;
-  sum += b[1 + w.nx] * xb1 * yb1;
-  return sum / T(4);
+  const T r0[2] = {b[0], b[1]}, r1[2] = {b[w.nx], b[w.nx + 1]};
+  return bilinear_sum2d<T>(r0, r1, fx, fy);
 }
 
 // GridInterpolate3D / 2D (Common/Grid.c:353-411), order k, j, i

@@ -80,17 +80,70 @@ __device__ __forceinline__ T curv3d_at(const T* __restrict__ p, int Y, int Z, co
   return curv3d_planes<T>(p - Z, p, p + Z, Y, r);
 }
 
-template <typename T>
-__device__ __forceinline__ T curv2d_at(const T* __restrict__ p, int Y, T dx, T dy) {
-  const T px = (p[1] - p[-1]) / (T(2.) * dx);
-  const T py = (p[Y] - p[-Y]) / (T(2.) * dy);
+// GridFunction2D_Curv (Common/Grid.c:231-254) at p (row stride Y), its five
+// divisions by the spacings' terms left to quot(a, d, which); NaN where the
+// gradient is zero or a value is not finite.  Written out operation by
+// operation (contraction off, fma where written), so that every kernel gives
+// the same bits.
+template <typename T, typename Ptr, typename Quot>
+__device__ __forceinline__ T curv2d_sum(Ptr p, int Y, T dx, T dy, Quot quot) {
+#pragma clang fp contract(off)
+  const T px = quot(p[1] - p[-1], T(2.) * dx, 0);
+  const T py = quot(p[Y] - p[-Y], T(2.) * dy, 1);
   const T px2 = px * px, py2 = py * py;
-  const T pxx = (p[-1] - T(2.) * p[0] + p[1]) / (dx * dx);
-  const T pyy = (p[-Y] - T(2.) * p[0] + p[Y]) / (dy * dy);
-  const T pxy = (p[-Y - 1] + p[Y + 1] - p[Y - 1] - p[-Y + 1]) / (T(4.) * dx * dy);
-  T k = grad_pow3_div<T>(pxx * py2 - T(2.) * px * py * pxy + pyy * px2, px2 + py2);
-  if (k != k) k = T(0);
-  return k;
+  const T pxx = quot(fma(T(-2.), p[0], p[-1]) + p[1], dx * dx, 2);
+  const T pyy = quot(fma(T(-2.), p[0], p[-Y]) + p[Y], dy * dy, 3);
+  const T pxy = quot(p[-Y - 1] + p[Y + 1] - p[Y - 1] - p[-Y + 1], T(4.) * dx * dy, 4);
+  const T c = fma(pyy, px2, fma(pxx, py2, -(T(2.) * px * py * pxy)));
+  return grad_pow3_div<T>(c, fma(px, px, py2));
+}
+
+template <typename T, typename Ptr>
+__device__ __forceinline__ T curv2d_at(Ptr p, int Y, T dx, T dy) {
+  const T k = curv2d_sum<T>(p, Y, dx, dy, [](T a, T d, int) { return a / d; });
+  return k != k ? T(0) : k;
+}
+
+// rounded reciprocals of curv2d_sum's divisors, for curv2d_recip_at; all 0
+// where one of them or its divisor is not a normal number
+template <typename T>
+struct Curv2R {
+  T r[5];
+};
+template <typename T>
+inline Curv2R<T> curv2d_recips(T dx, T dy) {
+  const T d[5] = {T(2.) * dx, T(2.) * dy, dx * dx, dy * dy, T(4.) * dx * dy};
+  Curv2R<T> c;
+  bool normal = true;
+  for (int q = 0; q < 5; ++q) {
+    c.r[q] = T(1) / d[q];
+    normal = normal && __builtin_isnormal(d[q]) && __builtin_isnormal(c.r[q]);
+  }
+  for (int q = 0; q < 5 && !normal; ++q) c.r[q] = T(0);
+  return c;
+}
+
+// The same values as curv2d_at, each quotient a / d by the rounded reciprocal
+// r of d and one correction step (P. Markstein, "Computation of elementary
+// functions on the IBM RISC System/6000 processor", 1990):
+//   t = a r,  a / d = t + (a - t d) r
+// with both sums fused, which rounds as the division does (the same for all
+// 2^23 FP32 mantissas of a with each of 1500 divisors, and for 4e8 FP64
+// pairs; a below 2^-102, FP64 2^-969, may be a rounding off, its remainder
+// being subnormal).  Three operations where a division is about eleven: 256
+// FP64 cells of edges 64 to 512 take 249 us a step, with divisions 275.
+// Where it does not hold (a value that is not finite, a quotient past the
+// largest number) it gives NaN, and the node is done again with divisions.
+template <typename T, typename Ptr>
+__device__ __forceinline__ T curv2d_recip_at(Ptr p, int Y, T dx, T dy, const Curv2R<T>& c) {
+  if (c.r[0] != T(0)) {
+    const T k = curv2d_sum<T>(p, Y, dx, dy, [&](T a, T d, int q) {
+      const T t = a * c.r[q];
+      return fma(fma(-t, d, a), c.r[q], t);
+    });
+    if (k == k) return k;
+  }
+  return curv2d_at<T>(p, Y, dx, dy);
 }
 
 // Least-squares fit c0 + c1 a + c2 b + c3 a^2 + c4 ab + c5 b^2 over the 9x9

@@ -9,8 +9,10 @@
 // corners come from there (a node whose stencil leaves the halo, a departure
 // of 2 cells or more, gathers from memory).  The new phi of the area goes to
 // LDS too, and the curvature of the nodes inside its outer layer is taken
-// from there; those 62 x (4 R - 2) nodes are the tile's output, the outer layer being worked by the neighbouring tiles too, with the same
-// bits.  So phi is written once and not read back.
+// from there; those 62 x (4 R - 2) nodes are the tile's output, the outer
+// layer being worked by the neighbouring tiles too, with the same bits.  So
+// phi is written once and not read back.  phi and kappa have the bits of the
+// separate SL and curvature kernels.
 //
 // What it replaces read every stencil value with its own gather (about 20
 // vector loads per node, the texture path's limit) and phi again for the
@@ -47,35 +49,6 @@ struct Step2Lds {
 // flat load of the two
 template <typename T>
 using lds_cptr = const __attribute__((address_space(3))) T*;
-
-// Bilinear2D (Common/Grid.c:190-212) from the rows y and y + 1: the (2x-1)
-// form, x outer, y inner, / 4, with every product-sum contracted
-template <typename T>
-__device__ __forceinline__ T bilinear_sum2d(const T r0[2], const T r1[2], double fx, double fy) {
-#pragma clang fp contract(off)
-  const T xf = (T)(2. * fx - 1.), yf = (T)(2. * fy - 1.);
-  const T xb0 = T(1) - xf, xb1 = T(1) + xf, yb0 = T(1) - yf, yb1 = T(1) + yf;
-  T sum = (r0[0] * xb0) * yb0;
-  sum = fma(r1[0] * xb0, yb1, sum);
-  sum = fma(r0[1] * xb1, yb0, sum);
-  sum = fma(r1[1] * xb1, yb1, sum);
-  return sum / T(4);
-}
-
-// GridFunction2D_Curv (Common/Grid.c:231-254) at p (row stride Y) with the
-// reciprocal spacings of curv_recips
-template <typename T>
-__device__ __forceinline__ T curv2d_recip(const T* p, int Y, const CurvR<T>& r) {
-  const T px = (p[1] - p[-1]) * r.x2;
-  const T py = (p[Y] - p[-Y]) * r.y2;
-  const T px2 = px * px, py2 = py * py;
-  const T pxx = (p[-1] - T(2.) * p[0] + p[1]) * r.xx;
-  const T pyy = (p[-Y] - T(2.) * p[0] + p[Y]) * r.yy;
-  const T pxy = (p[-Y - 1] + p[Y + 1] - p[Y - 1] - p[-Y + 1]) * r.xy;
-  T k = grad_pow3_div<T>(pxx * py2 - T(2.) * px * py * pxy + pyy * px2, px2 + py2);
-  if (k != k) k = T(0);
-  return k;
-}
 
 // the SL value of interior node (i, j) of a window whose velocity has the
 // same window; (x0, y0) the area's first node
@@ -160,7 +133,7 @@ __device__ __forceinline__ T step2d_node(const T* __restrict__ phi0, const T* __
 // the window.  Every thread of the block calls it; it ends on a barrier.
 template <typename T, int INTERP, int BT, int R>
 __device__ __forceinline__ void step2d_tile(const T* __restrict__ phi0, T* __restrict__ phi, T* __restrict__ kappa,
-                                            const T* __restrict__ vel, const SLP& P, const CurvR<T>& cr, int ox,
+                                            const T* __restrict__ vel, const SLP& P, T dx, T dy, const Curv2R<T>& cr, int ox,
                                             int oy, Step2Lds<T, R>& S) {
   typedef Step2<R> G;
   const int nx = P.w.nx, ny = P.w.ny;
@@ -213,7 +186,7 @@ __device__ __forceinline__ void step2d_tile(const T* __restrict__ phi0, T* __res
       if (row < 1 || row > G::OY || j >= ny) continue;
       T k = T(0);
       if (i >= 1 && i <= nx - 2 && j >= 1 && j <= ny - 2)
-        k = curv2d_recip<T>(S.out + row * S2_TX + threadIdx.x, S2_TX, cr);
+        k = curv2d_recip_at<T>((lds_cptr<T>)S.out + row * S2_TX + threadIdx.x, S2_TX, dx, dy, cr);
       phi[j * nx + i] = S.out[row * S2_TX + threadIdx.x];
       kappa[j * nx + i] = k;
     }

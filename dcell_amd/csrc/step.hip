@@ -19,9 +19,9 @@ int sl_params(const dcl_window* win, const dcl_velocity* vel, double dt, SLP& P)
 template <typename T, int INTERP, int BT, int R>
 __global__ __launch_bounds__(Step2<R>::NT) void step2d_k(const T* __restrict__ phi0, T* __restrict__ phi,
                                                          T* __restrict__ kappa, const T* __restrict__ vel, SLP P,
-                                                         CurvR<T> cr) {
+                                                         T dx, T dy, Curv2R<T> cr) {
   __shared__ Step2Lds<T, R> S;
-  step2d_tile<T, INTERP, BT, R>(phi0, phi, kappa, vel, P, cr, (int)blockIdx.x * Step2<R>::OX,
+  step2d_tile<T, INTERP, BT, R>(phi0, phi, kappa, vel, P, dx, dy, cr, (int)blockIdx.x * Step2<R>::OX,
                                 (int)blockIdx.y * Step2<R>::OY, S);
 }
 
@@ -37,17 +37,18 @@ static dim3 step2d_grid(const KWin& w) {
 // 8.1 / 6.9 / 8.5, 768 15.5 / 13.0 / 11.7, 1024 23.0 / 18.8 / 17.8; FP32 and
 // the trilinear scheme cross at the same sizes).
 template <typename T, int INTERP, int BT>
-static int step2d_launch(const T* phi0, T* phi, T* kappa, const T* vel, const SLP& P, const CurvR<T>& cr,
+static int step2d_launch(const T* phi0, T* phi, T* kappa, const T* vel, const SLP& P, T dx, T dy,
                          hipStream_t s) {
+  const Curv2R<T> cr = curv2d_recips<T>(dx, dy);
   // at least `halves` half blocks per CU
   auto fills = [](dim3 g, int halves) { return 2 * (int64_t)g.x * g.y >= (int64_t)halves * device_cus(); };
   const dim3 block(S2_TX, S2_TY);
   if (fills(step2d_grid<4>(P.w), 5))
-    hipLaunchKernelGGL((step2d_k<T, INTERP, BT, 4>), step2d_grid<4>(P.w), block, 0, s, phi0, phi, kappa, vel, P, cr);
+    hipLaunchKernelGGL((step2d_k<T, INTERP, BT, 4>), step2d_grid<4>(P.w), block, 0, s, phi0, phi, kappa, vel, P, dx, dy, cr);
   else if (fills(step2d_grid<2>(P.w), 3))
-    hipLaunchKernelGGL((step2d_k<T, INTERP, BT, 2>), step2d_grid<2>(P.w), block, 0, s, phi0, phi, kappa, vel, P, cr);
+    hipLaunchKernelGGL((step2d_k<T, INTERP, BT, 2>), step2d_grid<2>(P.w), block, 0, s, phi0, phi, kappa, vel, P, dx, dy, cr);
   else
-    hipLaunchKernelGGL((step2d_k<T, INTERP, BT, 1>), step2d_grid<1>(P.w), block, 0, s, phi0, phi, kappa, vel, P, cr);
+    hipLaunchKernelGGL((step2d_k<T, INTERP, BT, 1>), step2d_grid<1>(P.w), block, 0, s, phi0, phi, kappa, vel, P, dx, dy, cr);
   DCL_LAUNCHED("step2d");
   return 0;
 }
@@ -57,15 +58,15 @@ static int step2d(const void* phi0, void* phi, void* kappa, const dcl_window* wi
                   int interp, int backtrace, hipStream_t s) {
   SLP P;
   sl_params(win, vel, dt, P);
-  const CurvR<T> cr = curv_recips<T>(win->d.x, win->d.y, 1.0);
+  const T dx = (T)win->d.x, dy = (T)win->d.y;
   const T* p0 = static_cast<const T*>(phi0);
   const T* v = static_cast<const T*>(vel->data);
   T* p = static_cast<T*>(phi);
   T* k = static_cast<T*>(kappa);
-  if (interp == DCL_CUBIC && backtrace == DCL_RK2) return step2d_launch<T, DCL_CUBIC, DCL_RK2>(p0, p, k, v, P, cr, s);
-  if (interp == DCL_CUBIC) return step2d_launch<T, DCL_CUBIC, DCL_EULER>(p0, p, k, v, P, cr, s);
-  if (backtrace == DCL_RK2) return step2d_launch<T, DCL_LINEAR, DCL_RK2>(p0, p, k, v, P, cr, s);
-  return step2d_launch<T, DCL_LINEAR, DCL_EULER>(p0, p, k, v, P, cr, s);
+  if (interp == DCL_CUBIC && backtrace == DCL_RK2) return step2d_launch<T, DCL_CUBIC, DCL_RK2>(p0, p, k, v, P, dx, dy, s);
+  if (interp == DCL_CUBIC) return step2d_launch<T, DCL_CUBIC, DCL_EULER>(p0, p, k, v, P, dx, dy, s);
+  if (backtrace == DCL_RK2) return step2d_launch<T, DCL_LINEAR, DCL_RK2>(p0, p, k, v, P, dx, dy, s);
+  return step2d_launch<T, DCL_LINEAR, DCL_EULER>(p0, p, k, v, P, dx, dy, s);
 }
 
 // the fused 2D step stages the velocity at phi's nodes; its grid's second

@@ -13,6 +13,7 @@ import torch
 import oracle as O
 import dcell_amd as D
 from dcell_amd import configs
+from dcell_amd.batch import Batch
 from helpers import owin, random_velocity, rel_max, rounded, smooth_field, to_dev, to_np
 
 pytestmark = pytest.mark.gpu
@@ -299,9 +300,8 @@ def test_levelset_step_planes_equal_per_node(dev, dtype, dim):
 def test_levelset_step_2d_tiles(dev, dtype, interp, bt, n, layout):
     """The fused 2D step around its tile edges, at each number of rows per
     thread, with every velocity layout (planes, (u, v), (p, u, v)) and
-    departures on both sides of the staged halo: phi against the oracle, kappa
-    against the curvature kernel on the same phi within the rounding of the
-    terms of its sum (33 unit roundoffs per evaluation)."""
+    departures on both sides of the staged halo: phi against the oracle and bit
+    for bit the SL kernel's, kappa the curvature kernel's on that phi."""
     rng = np.random.default_rng(n[0] + n[1])
     h = 1.0 / (max(n) - 1)
     win = D.GridWindow((3, -2, 0), (n[0], n[1], 1), (h, 1.2 * h, h))
@@ -319,19 +319,57 @@ def test_levelset_step_2d_tiles(dev, dtype, interp, bt, n, layout):
     phi, kap = D.levelset_step(to_dev(phi0, dtype), dvel, win, dt, interp, bt, **kw)
     ref = O.sl_advect(phi0, vel, owin(win), dt, IM[interp], BM[bt])
     assert rel_max(to_np(phi), ref) <= TOL[dtype]
-    other = to_np(D.curvature(phi, win))
-    p = to_np(phi)
-    px, py = (p[1:-1, 2:] - p[1:-1, :-2]) / (2 * win.d[0]), (p[2:, 1:-1] - p[:-2, 1:-1]) / (2 * win.d[1])
-    pxx = (p[1:-1, 2:] - 2 * p[1:-1, 1:-1] + p[1:-1, :-2]) / win.d[0] ** 2
-    pyy = (p[2:, 1:-1] - 2 * p[1:-1, 1:-1] + p[:-2, 1:-1]) / win.d[1] ** 2
-    pxy = (p[2:, 2:] + p[:-2, :-2] - p[2:, :-2] - p[:-2, 2:]) / (4 * win.d[0] * win.d[1])
-    # the sums of p are rounded in the kernels' precision, the same in both
-    mag = (np.abs(pxx) * py ** 2 + 2 * np.abs(px * py * pxy) + np.abs(pyy) * px ** 2) / (px ** 2 + py ** 2) ** 1.5
-    lost = 4 * np.abs(p).max() * (1 / win.d[0] ** 2 + 1 / win.d[1] ** 2) / np.sqrt(px ** 2 + py ** 2)
-    u = 2.0 ** (-53 if dtype == torch.float64 else -24)
-    diff = np.abs(to_np(kap) - other)
-    assert diff[0].max() == diff[-1].max() == diff[:, 0].max() == diff[:, -1].max() == 0
-    assert np.all(diff[1:-1, 1:-1] <= 66 * u * (mag + u * lost))
+    assert torch.equal(phi, D.advect_sl(to_dev(phi0, dtype), dvel, win, dt, interp, bt, **kw))
+    assert torch.equal(kap, D.curvature(phi, win))
+
+
+def _same(a, b):
+    """Equal values, NaN where the other is NaN."""
+    return bool(((a == b) | (a.isnan() & b.isnan())).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+@pytest.mark.parametrize("interp,bt", [("cubic", "rk2"), ("linear", "euler"), ("linear", "rk2"), ("cubic", "euler")])
+@pytest.mark.parametrize("values", ["smooth", "flat", "odd"])
+@pytest.mark.parametrize("h", [(0.013, 0.021), (1e-30, 1e-30), (1e22, 1e-3)])
+def test_2d_entry_points_share_bits(dev, dtype, interp, bt, values, h):
+    """levelset_step, advect_sl then curvature, Batch.step and Batch.band_step
+    give one field the same phi and kappa: smooth, with zero gradients, and
+    with infinities, NaN and the largest numbers in it; with spacings whose
+    squares leave FP32's range."""
+    rng = np.random.default_rng(5)
+    n = (130, 97)
+    win = D.GridWindow((3, -2, 0), (n[0], n[1], 1), h + (1.0,))
+    y, x = np.meshgrid(np.arange(float(n[1])), np.arange(float(n[0])), indexing="ij")
+    phi0 = np.hypot(x - 0.4 * n[0], y - 0.55 * n[1]) - 0.3 * min(n)
+    if values == "flat":
+        phi0 = np.round(phi0 / 8)
+    if values == "odd":
+        for v in (np.inf, -np.inf, np.nan, torch.finfo(dtype).max, -0.0):
+            phi0[rng.random(phi0.shape) < 0.02] = v
+    vel = np.stack([np.sin(0.11 * y + 0.05 * x), np.cos(0.07 * x - 0.1 * y)], axis=-1) + rng.normal(size=2)
+    dphi0, dvel = to_dev(phi0, dtype), to_dev(vel, dtype)
+    dt = 0.9 * min(h)
+    phi, kap = D.levelset_step(dphi0, dvel, win, dt, interp, bt)
+    two = D.advect_sl(dphi0, dvel, win, dt, interp, bt)
+    assert _same(phi, two) and _same(kap, D.curvature(two, win))
+    b = Batch([win, win], dtype=dtype, interp=interp, backtrace=bt)
+    b.set_dt([dt, dt])
+    bphi, bkap, pair, pvel = b.new_field(), b.new_field(), b.new_field(), b.new_field(2)
+    for c in range(2):
+        b.cell(pair, c).copy_(dphi0)
+        b.cell(pvel, c, 2).copy_(dvel)
+    b.step(pair, bphi, bkap, pvel)
+    for c in range(2):
+        assert _same(b.cell(bphi, c), phi) and _same(b.cell(bkap, c), kap)
+    # band mode at the interior nodes of cell 1, over the step's phi
+    band = np.stack([x[2:-2, 2:-2].ravel() + 3, y[2:-2, 2:-2].ravel() - 2, 0 * x[2:-2, 2:-2].ravel(),
+                     1 + 0 * x[2:-2, 2:-2].ravel()], axis=1).astype(np.int32)
+    bphi2, bkap2 = pair.clone(), torch.zeros_like(bkap)
+    b.band_step(pair, bphi2, bkap2, pvel, torch.from_numpy(band).to("cuda:0"))
+    assert _same(b.cell(bphi2, 1), phi)
+    assert _same(b.cell(bkap2, 1)[2:-2, 2:-2], kap[2:-2, 2:-2])
+    b.close()
 
 
 def test_zalesak_c1_revolution_fp64(dev):
