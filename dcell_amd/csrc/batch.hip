@@ -11,7 +11,7 @@
 // configurations, and the ring columns' z-chunk is chosen per cell-size
 // class; dcl_batch_autotune times them on the caller's buffers and keeps the
 // fastest.  2D cells: SL and curvature of a tile in one pass (dcl_step2d.hpp),
-// one launch.  Band mode
+// one launch (two where kappa takes memory of phi0 or the velocity).  Band mode
 // (dcl_batch_band_step): only the listed nodes of every cell, as the
 // reference's band loop (LevelSetMethod/AdvectSL.c:23-89), one thread per
 // node over the packed band list.
@@ -210,8 +210,8 @@ __global__ __launch_bounds__(shape_of(S).tx * shape_of(S).ty) void batch_curv_k(
   });
 }
 
-// 2D cells: SL and curvature of one tile after another (nodes outside
-// [2, n-3] copy phi0, as in the dense 2D step)
+// 2D cells: SL and, unless kappa is NULL, curvature of one tile after another
+// (nodes outside [2, n-3] copy phi0, as in the dense 2D step)
 template <typename T, int INTERP, int BT>
 __global__ __launch_bounds__(Step2<T2R>::NT) void batch2d_step_k(const T* __restrict__ phi0, T* __restrict__ phi,
                                                                  T* __restrict__ kappa, const T* __restrict__ vel,
@@ -237,6 +237,23 @@ template <typename T>
 __device__ __forceinline__ T curv2d_node(const T* __restrict__ p, const BCell& c, int i, int j) {
   if (i < 1 || i > c.nx - 2 || j < 1 || j > c.ny - 2) return T(0);
   return curv2d_at<T>(p + j * c.nx + i, c.nx, (T)c.dx, (T)c.dy);
+}
+
+// 2D cells: the curvature by itself, over the same tiles
+template <typename T>
+__global__ __launch_bounds__(Step2<T2R>::NT) void batch2d_curv_k(const T* __restrict__ phi, T* __restrict__ kappa,
+                                                                 const BCell* __restrict__ cells,
+                                                                 const int4* __restrict__ tiles,
+                                                                 const int* __restrict__ bounds,
+                                                                 WorkQ* __restrict__ q, int k) {
+  claim_tiles(q, bounds, k, [&](int t) {
+    const int4 tl = tiles[t];
+    const BCell c = cells[tl.x];
+    const int i = tl.y + threadIdx.x, j1 = min(tl.z + T2Y, c.ny);
+    if ((int)threadIdx.x >= T2X || i >= c.nx) return;
+    for (int j = tl.z + threadIdx.y; j < j1; j += S2_TY)
+      kappa[c.phi_off + j * c.nx + i] = curv2d_node<T>(phi + c.phi_off, c, i, j);
+  });
 }
 
 // Band mode: entry b of the packed list is {x, y, z, cell} in the cell's
@@ -436,7 +453,8 @@ static int grid_blocks(dcl_batch b, int occ) {
 }
 
 // the two launches of one step with configuration (s, occ); 2D: one (kcv is
-// NULL)
+// NULL) that writes kappa too, or two where kappa shares memory with what the
+// first reads
 struct Plan {
   const void* ksl;
   const void* kcv;
@@ -450,7 +468,7 @@ struct Plan {
   int k;
 };
 
-static int make_plan(dcl_batch b, int s, int occ, Plan& p) {
+static int make_plan(dcl_batch b, int s, int occ, const void* phi0, const void* kappa, const void* vel, Plan& p) {
   const bool f64 = b->precision == DCL_F64;
   p.grid = dim3(grid_blocks(b, occ));
   p.k = b->claim;
@@ -462,7 +480,10 @@ static int make_plan(dcl_batch b, int s, int occ, Plan& p) {
     p.tsl = p.tcv = b->tiles[0];
     p.bsl_bounds = p.bcv_bounds = b->bounds[0];
     p.ksl = f64 ? sl_kernel<double>(b->interp, b->backtrace, 2, 0) : sl_kernel<float>(b->interp, b->backtrace, 2, 0);
+    const int64_t bytes = b->phi_off[b->ncells] * (f64 ? 8 : 4);
     p.kcv = nullptr;
+    if (overlap(kappa, bytes, phi0, bytes) || overlap(kappa, bytes, vel, 2 * bytes))
+      p.kcv = f64 ? (const void*)&batch2d_curv_k<double> : (const void*)&batch2d_curv_k<float>;
     return 0;
   }
   const int cs = s % NBASE;
@@ -492,17 +513,18 @@ static int make_plan(dcl_batch b, int s, int occ, Plan& p) {
 // the arguments of a plan's launches (pointers to the members)
 struct PlanArgs {
   const void *phi0, *cphi, *vel;
-  void *phi, *kappa;
+  void *phi, *kappa, *skappa;  // skappa: kappa of the 2D launch
   const BCell* cells;
   Plan p;
   void* sl[9];
   void* cv[7];
   PlanArgs(dcl_batch b, const Plan& plan, const void* phi0_, void* phi_, void* kappa_, const void* vel_)
-      : phi0(phi0_), cphi(phi_), vel(vel_), phi(phi_), kappa(kappa_), cells(b->cells), p(plan) {
+      : phi0(phi0_), cphi(phi_), vel(vel_), phi(phi_), kappa(kappa_), skappa(plan.kcv ? nullptr : kappa_),
+        cells(b->cells), p(plan) {
     int n = 0;
     sl[n++] = &phi0;
     sl[n++] = &phi;
-    if (!p.kcv) sl[n++] = &kappa;
+    if (b->dim == 2) sl[n++] = &skappa;
     sl[n++] = &vel;
     sl[n++] = &cells;
     sl[n++] = &p.tsl;
@@ -519,7 +541,7 @@ struct PlanArgs {
 static int batch_launch(dcl_batch b, int s, int occ, const void* phi0, void* phi, void* kappa, const void* vel,
                         hipStream_t st) {
   Plan p;
-  DCL_TRY(make_plan(b, s, occ, p));
+  DCL_TRY(make_plan(b, s, occ, phi0, kappa, vel, p));
   PlanArgs a(b, p, phi0, phi, kappa, vel);
   DCL_HIP(hipLaunchKernel(p.ksl, p.grid, p.bsl, a.sl, 0, st));
   if (p.kcv) DCL_HIP(hipLaunchKernel(p.kcv, p.grid, p.bcv, a.cv, 0, st));
@@ -828,7 +850,7 @@ extern "C" int dcl_batch_graph_create(dcl_batch b, const void* phi0, void* phi, 
   DCL_TRY(check_step(b, phi0, phi, kappa, vel));
   if (!graph_exec) return set_error(DCL_ERR_ARG_NULL, "graph_exec is NULL");
   Plan p;
-  DCL_TRY(make_plan(b, b->shape, b->occ, p));
+  DCL_TRY(make_plan(b, b->shape, b->occ, phi0, kappa, vel, p));
   PlanArgs a(b, p, phi0, phi, kappa, vel);
   hipGraph_t g;
   DCL_HIP(hipGraphCreate(&g, 0));

@@ -28,6 +28,12 @@ int check_window(const dcl_window* w, const char* name, int min_n, int dof = 1);
 int check_velocity(const dcl_velocity* v, int dim, bool planes = false);
 int check_precision(int precision);
 
+// whether two buffers have memory in common
+inline bool overlap(const void* a, int64_t abytes, const void* b, int64_t bbytes) {
+  const char *p = static_cast<const char*>(a), *q = static_cast<const char*>(b);
+  return p < q + bbytes && q < p + abytes;
+}
+
 inline unsigned grid1d(int64_t n, int block) { return (unsigned)((n + block - 1) / block); }
 
 // compute units of the current device (queried once per device; 256 if the

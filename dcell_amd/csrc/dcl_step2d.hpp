@@ -130,7 +130,7 @@ __device__ __forceinline__ T step2d_node(const T* __restrict__ phi0, const T* __
 }
 
 // one tile: output nodes (ox .. ox + OX - 1, oy .. oy + OY - 1) clipped to
-// the window.  Every thread of the block calls it; it ends on a barrier.
+// the window; kappa may be NULL (phi only).  Every thread of the block calls it; it ends on a barrier.
 template <typename T, int INTERP, int BT, int R>
 __device__ __forceinline__ void step2d_tile(const T* __restrict__ phi0, T* __restrict__ phi, T* __restrict__ kappa,
                                             const T* __restrict__ vel, const SLP& P, T dx, T dy, const Curv2R<T>& cr, int ox,
@@ -184,10 +184,11 @@ __device__ __forceinline__ void step2d_tile(const T* __restrict__ phi0, T* __res
     for (int r = 0; r < R; ++r) {
       const int row = threadIdx.y + S2_TY * r, j = y0 + row;
       if (row < 1 || row > G::OY || j >= ny) continue;
+      phi[j * nx + i] = S.out[row * S2_TX + threadIdx.x];
+      if (!kappa) continue;
       T k = T(0);
       if (i >= 1 && i <= nx - 2 && j >= 1 && j <= ny - 2)
         k = curv2d_recip_at<T>((lds_cptr<T>)S.out + row * S2_TX + threadIdx.x, S2_TX, dx, dy, cr);
-      phi[j * nx + i] = S.out[row * S2_TX + threadIdx.x];
       kappa[j * nx + i] = k;
     }
   }

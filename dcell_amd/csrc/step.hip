@@ -1,7 +1,8 @@
 // step.hip -- one dense level-set update: SL step phi0 -> phi followed by
 // the 19-point (3D) / 9-point (2D) curvature of the new phi.  3D: the SL and
 // the curvature kernel one after the other.  2D with the velocity on phi's
-// window: one fused launch (dcl_step2d.hpp).
+// window: one fused launch (dcl_step2d.hpp), unless kappa takes memory of phi0
+// or the velocity, which the fused launch still reads when it writes kappa.
 #include "dcl_host.hpp"
 #include "dcl_step2d.hpp"
 
@@ -71,8 +72,13 @@ static int step2d(const void* phi0, void* phi, void* kappa, const dcl_window* wi
 
 // the fused 2D step stages the velocity at phi's nodes; its grid's second
 // dimension holds at most 65535 tiles (two rows each where they are smallest)
-static bool step2d_takes(const dcl_window& w, const dcl_window& v) {
-  return w.n.z < 2 && v.p.x == w.p.x && v.p.y == w.p.y && v.n.x == w.n.x && v.n.y == w.n.y && w.n.y <= 100000;
+static bool step2d_takes(const void* phi0, const void* kappa, const dcl_window& w, const dcl_velocity& vel,
+                         int precision) {
+  const dcl_window& v = vel.win;
+  if (w.n.z >= 2 || v.p.x != w.p.x || v.p.y != w.p.y || v.n.x != w.n.x || v.n.y != w.n.y || w.n.y > 100000)
+    return false;
+  const int64_t bytes = win_nodes(w) * (precision == DCL_F64 ? 8 : 4);
+  return !overlap(kappa, bytes, phi0, bytes) && !overlap(kappa, bytes, vel.data, bytes * (vel.dof == 1 ? 2 : vel.dof));
 }
 }  // namespace dcl
 
@@ -86,7 +92,7 @@ extern "C" int dcl_levelset_step(const void* phi0, void* phi, void* kappa, const
   if (kappa == phi || kappa == phi0)
     return set_error(DCL_ERR_ARG_WRONG, "kappa must not alias phi or phi0");
   hipStream_t s = as_stream(stream);
-  if (step2d_takes(*win, vel->win))
+  if (step2d_takes(phi0, kappa, *win, *vel, precision))
     return precision == DCL_F64 ? step2d<double>(phi0, phi, kappa, win, vel, dt, interp, backtrace, s)
                                 : step2d<float>(phi0, phi, kappa, win, vel, dt, interp, backtrace, s);
   DCL_TRY(sl_launch(phi0, phi, win, vel, nullptr, 0, nullptr, dt, precision, interp, backtrace, s));

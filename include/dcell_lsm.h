@@ -430,7 +430,8 @@ int dcl_batch_set_class_zchunk(dcl_batch batch, int cls, int zchunk);
  * count and its ring z-chunk; any pointer may be NULL */
 int dcl_batch_get_classes(dcl_batch batch, int32_t max_edge[DCL_BATCH_CLASSES],
                           int32_t cells[DCL_BATCH_CLASSES], int32_t zchunk[DCL_BATCH_CLASSES]);
-/* one step phi0 -> phi, kappa(phi) for every cell */
+/* one step phi0 -> phi, kappa(phi) for every cell.  kappa may take the memory
+ * of vel, or part of phi0's: in 2D the curvature is then a launch of its own. */
 int dcl_batch_step(dcl_batch batch, const void *phi0, void *phi, void *kappa, const void *vel,
                    void *stream);
 /* Band mode, the band loop of LevelSetAdvectSL_2D / _3D
@@ -452,7 +453,7 @@ int dcl_batch_autotune(dcl_batch batch, const void *phi0, void *phi, void *kappa
                        const void *vel, int reps, double *ms_table, double *zc_table,
                        double *claim_table, double *best_ms, void *stream);
 /* One step with these buffers recorded as an instantiated hipGraph (two
- * kernel nodes, in 2D one); launch it with dcl_batch_graph_launch. */
+ * kernel nodes, in 2D one as dcl_batch_step); launch it with dcl_batch_graph_launch. */
 int dcl_batch_graph_create(dcl_batch batch, const void *phi0, void *phi, void *kappa,
                            const void *vel, void **graph_exec);
 int dcl_batch_graph_launch(void *graph_exec, void *stream);

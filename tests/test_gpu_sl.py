@@ -372,6 +372,52 @@ def test_2d_entry_points_share_bits(dev, dtype, interp, bt, values, h):
     b.close()
 
 
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+@pytest.mark.parametrize("planes", [False, True])
+def test_2d_kappa_in_the_inputs_memory(dev, dtype, planes):
+    """kappa written over the velocity, or over a part of phi0: the step and
+    the batch (a graph of it too) give what they give with kappa apart."""
+    rng = np.random.default_rng(8)
+    n = (500, 430)
+    win = D.GridWindow((0, 0, 0), (n[0], n[1], 1), (0.01, 0.01, 0.01))
+    y, x = np.meshgrid(np.arange(float(n[1])), np.arange(float(n[0])), indexing="ij")
+    phi0 = to_dev(np.hypot(x - 0.4 * n[0], y - 0.5 * n[1]) - 90 + np.sin(0.3 * x), dtype)
+    vel = to_dev(np.stack([np.sin(0.11 * y), np.cos(0.07 * x)], axis=0 if planes else -1) + rng.normal(), dtype)
+    dt, nodes = 0.008, win.nodes
+    ref = [t.clone() for t in D.levelset_step(phi0, vel, win, dt, "cubic", "rk2", planes=planes)]
+
+    def check(phi, kappa):
+        assert torch.equal(phi.reshape(-1), ref[0].reshape(-1)) and torch.equal(kappa.reshape(-1), ref[1].reshape(-1))
+
+    v = vel.clone()
+    check(*D.levelset_step(phi0, v, win, dt, "cubic", "rk2", planes=planes,
+                           out_kappa=v.reshape(-1)[nodes // 2:][:nodes].view(win.shape)))
+    room = torch.zeros(2 * nodes, dtype=dtype, device="cuda:0")
+    both = room[:nodes].view(win.shape).copy_(phi0)
+    check(*D.levelset_step(both, vel, win, dt, "cubic", "rk2", planes=planes,
+                           out_kappa=room[nodes // 3:][:nodes].view(win.shape)))
+    if planes:
+        return
+    b = Batch([win], dtype=dtype, interp="cubic", backtrace="rk2")
+    b.set_dt([dt])
+    v, phi = vel.clone().reshape(-1), b.new_field()
+    kap = v[nodes // 2:][:nodes]
+    b.step(phi0.reshape(-1), phi, kap, v)
+    check(phi, kap)
+    g = b.graph(phi0.reshape(-1), phi, kap, v)
+    for _ in range(3):
+        v.copy_(vel.reshape(-1))
+        phi.zero_()
+        Batch.launch(g)
+        check(phi, kap)
+    room.zero_()
+    both = room[:nodes].copy_(phi0.reshape(-1))
+    kap = room[nodes // 3:][:nodes]
+    b.step(both, phi, kap, vel.reshape(-1))
+    check(phi, kap)
+    b.close()
+
+
 def test_zalesak_c1_revolution_fp64(dev):
     """C1 (128^2 Zalesak disk, rigid rotation, dt = 1/628) for 157 steps (a
     quarter revolution) in reference mode (Euler + Bilinear2D) and config mode
