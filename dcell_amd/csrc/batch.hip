@@ -60,8 +60,9 @@ __host__ __device__ constexpr TileShape shape_of(int s) {
 }
 constexpr int NOCC = 3;
 constexpr int occ_of(int o) { return o == 0 ? 2 : o == 1 ? 4 : 8; }  // resident blocks per CU
-// 2D tiles: 62 x 14 nodes of 64 x 16 worked, four rows per thread
-constexpr int T2R = 4, T2X = Step2<T2R>::OX, T2Y = Step2<T2R>::OY;
+// 2D tiles: step2d_cols x t2y nodes (dcl_step2d.hpp), the rows per thread
+// chosen with the batch from all its tiles
+constexpr int t2y(int rows) { return S2_TY * rows - 2; }
 // cell-size classes (largest axis up to 48, up to 80, beyond) and the ring
 // z-chunks tried for each
 constexpr int NCLASS = DCL_BATCH_CLASSES;
@@ -212,22 +213,23 @@ __global__ __launch_bounds__(shape_of(S).tx * shape_of(S).ty) void batch_curv_k(
 
 // 2D cells: SL and, unless kappa is NULL, curvature of one tile after another
 // (nodes outside [2, n-3] copy phi0, as in the dense 2D step)
-template <typename T, int INTERP, int BT>
-__global__ __launch_bounds__(Step2<T2R>::NT) void batch2d_step_k(const T* __restrict__ phi0, T* __restrict__ phi,
+template <typename T, int INTERP, int BT, int R>
+__global__ __launch_bounds__(Step2<R>::NT) void batch2d_step_k(const T* __restrict__ phi0, T* __restrict__ phi,
                                                                  T* __restrict__ kappa, const T* __restrict__ vel,
                                                                  const BCell* __restrict__ cells,
                                                                  const int4* __restrict__ tiles,
                                                                  const int* __restrict__ bounds,
                                                                  WorkQ* __restrict__ q, int k) {
-  __shared__ Step2Lds<T, T2R> S;
+  __shared__ Step2Lds<T, R> S;
   claim_tiles(q, bounds, k, [&](int t) {
     const int4 tl = tiles[t];
     const BCell c = cells[tl.x];
     Curv2R<T> cr;
 #pragma unroll
     for (int q = 0; q < 5; ++q) cr.r[q] = (T)c.r2[q];
-    step2d_tile<T, INTERP, BT, T2R>(phi0 + c.phi_off, phi + c.phi_off, kappa + c.phi_off, vel + c.vel_off,
-                                    cell_slp<2>(c), (T)c.dx, (T)c.dy, cr, tl.y, tl.z, S);
+    step2d_tile<T, INTERP, BT, R>(phi0 + c.phi_off, phi + c.phi_off, kappa + c.phi_off, vel + c.vel_off,
+                                    cell_slp<2>(c), (T)c.dx, (T)c.dy, cr, tl.y, tl.z,
+                                 tl.w, S);
   });
 }
 
@@ -241,16 +243,16 @@ __device__ __forceinline__ T curv2d_node(const T* __restrict__ p, const BCell& c
 
 // 2D cells: the curvature by itself, over the same tiles
 template <typename T>
-__global__ __launch_bounds__(Step2<T2R>::NT) void batch2d_curv_k(const T* __restrict__ phi, T* __restrict__ kappa,
+__global__ __launch_bounds__(S2_TX * S2_TY) void batch2d_curv_k(const T* __restrict__ phi, T* __restrict__ kappa,
                                                                  const BCell* __restrict__ cells,
                                                                  const int4* __restrict__ tiles,
                                                                  const int* __restrict__ bounds,
-                                                                 WorkQ* __restrict__ q, int k) {
+                                                                 WorkQ* __restrict__ q, int k, int rows) {
   claim_tiles(q, bounds, k, [&](int t) {
     const int4 tl = tiles[t];
     const BCell c = cells[tl.x];
-    const int i = tl.y + threadIdx.x, j1 = min(tl.z + T2Y, c.ny);
-    if ((int)threadIdx.x >= T2X || i >= c.nx) return;
+    const int i = tl.y + threadIdx.x, j1 = min(tl.z + t2y(rows), c.ny);
+    if ((int)threadIdx.x >= tl.w || i >= c.nx) return;
     for (int j = tl.z + threadIdx.y; j < j1; j += S2_TY)
       kappa[c.phi_off + j * c.nx + i] = curv2d_node<T>(phi + c.phi_off, c, i, j);
   });
@@ -311,7 +313,11 @@ struct KTable {
     }
   }
   static const void* ring() { return (const void*)&batch_ring_k<T, INTERP, BT>; }
-  static const void* step2d() { return (const void*)&batch2d_step_k<T, INTERP, BT>; }
+  static const void* step2d(int rows) {
+    return rows == 4   ? (const void*)&batch2d_step_k<T, INTERP, BT, 4>
+           : rows == 2 ? (const void*)&batch2d_step_k<T, INTERP, BT, 2>
+                       : (const void*)&batch2d_step_k<T, INTERP, BT, 1>;
+  }
   static const void* band(int dim) {
     return dim == 3 ? (const void*)&batch_band_sl_k<T, 3, INTERP, BT>
                     : (const void*)&batch_band_sl_k<T, 2, INTERP, BT>;
@@ -330,11 +336,11 @@ static const void* curv_kernel(int s) {
   }
 }
 
-// SL kernels by kind: 0 tile gathers of shape s, 1 ring columns, 2 2D
-// tiles (the curvature with them), 3 band mode of dimension s
+// SL kernels by kind: 0 tile gathers of shape s, 1 ring columns, 2 2D tiles
+// of s rows per thread (the curvature with them), 3 band mode of dimension s
 template <typename K>
 static const void* sl_pick(int kind, int s) {
-  return kind == 0 ? K::sl(s) : kind == 1 ? K::ring() : kind == 2 ? K::step2d() : K::band(s);
+  return kind == 0 ? K::sl(s) : kind == 1 ? K::ring() : kind == 2 ? K::step2d(s) : K::band(s);
 }
 
 template <typename T>
@@ -361,6 +367,7 @@ struct dcl_batch_s {
   int ntiles[NBASE + 1] = {0};
   WorkQ* queues = nullptr;              // [0] the SL launch, [1] the curvature launch
   int shape = 1, occ = 1;
+  int rows2 = 4;                        // 2D: rows per thread
   int claim = 0;                        // tiles per claim of both launches (0: static stride)
   int zc[NCLASS] = {32, 32, 32};        // ring z-chunk per size class
   int cus = 256;
@@ -397,7 +404,7 @@ static int build_tiles(dcl_batch b, int s) {
   std::vector<double> cost;
   for (int c : order) {
     const dcl_window& w = b->wins[c];
-    const TileShape sh = two                ? TileShape{T2X, T2Y, 1}
+    const TileShape sh = two                ? TileShape{step2d_cols(w.n.x, b->rows2), t2y(b->rows2), 1}
                          : s == RING_LIST ? TileShape{RING_TX, RING_TY, b->zc[b->cls[c]]}
                                           : shape_of(s);
     const int halo = two ? 0 : s == RING_LIST ? 2 * RG_H : 2;
@@ -405,7 +412,7 @@ static int build_tiles(dcl_batch b, int s) {
     for (int z = 0; z < nz; z += sh.tz)
       for (int y = 0; y < w.n.y; y += sh.ty)
         for (int x = 0; x < w.n.x; x += sh.tx) {
-          t.push_back(make_int4(c, x, y, z));
+          t.push_back(make_int4(c, x, y, two ? sh.tx : z));
           cost.push_back((double)sh.tx * sh.ty * (std::min(sh.tz, nz - z) + halo));
         }
   }
@@ -465,7 +472,7 @@ struct Plan {
   const int* bcv_bounds;
   WorkQ* qsl;
   WorkQ* qcv;
-  int k;
+  int k, rows;  // rows: of a 2D tile per thread
 };
 
 static int make_plan(dcl_batch b, int s, int occ, const void* phi0, const void* kappa, const void* vel, Plan& p) {
@@ -479,7 +486,9 @@ static int make_plan(dcl_batch b, int s, int occ, const void* phi0, const void* 
     p.bsl = p.bcv = dim3(S2_TX, S2_TY);
     p.tsl = p.tcv = b->tiles[0];
     p.bsl_bounds = p.bcv_bounds = b->bounds[0];
-    p.ksl = f64 ? sl_kernel<double>(b->interp, b->backtrace, 2, 0) : sl_kernel<float>(b->interp, b->backtrace, 2, 0);
+    p.ksl = f64 ? sl_kernel<double>(b->interp, b->backtrace, 2, b->rows2)
+                : sl_kernel<float>(b->interp, b->backtrace, 2, b->rows2);
+    p.rows = b->rows2;
     const int64_t bytes = b->phi_off[b->ncells] * (f64 ? 8 : 4);
     p.kcv = nullptr;
     if (overlap(kappa, bytes, phi0, bytes) || overlap(kappa, bytes, vel, 2 * bytes))
@@ -517,7 +526,7 @@ struct PlanArgs {
   const BCell* cells;
   Plan p;
   void* sl[9];
-  void* cv[7];
+  void* cv[8];
   PlanArgs(dcl_batch b, const Plan& plan, const void* phi0_, void* phi_, void* kappa_, const void* vel_)
       : phi0(phi0_), cphi(phi_), vel(vel_), phi(phi_), kappa(kappa_), skappa(plan.kcv ? nullptr : kappa_),
         cells(b->cells), p(plan) {
@@ -531,7 +540,7 @@ struct PlanArgs {
     sl[n++] = &p.bsl_bounds;
     sl[n++] = &p.qsl;
     sl[n++] = &p.k;
-    void* c[7] = {&cphi, &kappa, &cells, &p.tcv, &p.bcv_bounds, &p.qcv, &p.k};
+    void* c[8] = {&cphi, &kappa, &cells, &p.tcv, &p.bcv_bounds, &p.qcv, &p.k, &p.rows};
     memcpy(cv, c, sizeof(cv));
   }
   PlanArgs(const PlanArgs&) = delete;
@@ -608,6 +617,14 @@ extern "C" int dcl_batch_create(int32_t ncells, const dcl_window* wins, int prec
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && cus > 0)
       b->cus = cus;
   }
+  if (dim == 2) {
+    int64_t t4 = 0, t2 = 0;
+    for (const dcl_window& w : b->wins) {
+      t4 += step2d_tiles(w.n.x, w.n.y, 4);
+      t2 += step2d_tiles(w.n.x, w.n.y, 2);
+    }
+    b->rows2 = step2d_rows(t4, t2, b->cus);
+  }
   void* p = nullptr;
   int rc = dcl_malloc(&p, sizeof(BCell) * ncells + 2 * sizeof(WorkQ));
   if (rc) {
@@ -674,7 +691,7 @@ extern "C" int dcl_batch_get_config(dcl_batch b, int* shape, int* occupancy, int
   if (!b) return set_error(DCL_ERR_ARG_NULL, "batch is NULL");
   if (shape) *shape = b->shape;
   if (occupancy) *occupancy = b->occ;
-  const TileShape sh = b->dim == 2 ? TileShape{T2X, T2Y, 1} : shape_of(b->shape);
+  const TileShape sh = b->dim == 2 ? TileShape{step2d_cols(b->wins[0].n.x, b->rows2), t2y(b->rows2), 1} : shape_of(b->shape);
   if (tile) {
     tile[0] = sh.tx;
     tile[1] = sh.ty;

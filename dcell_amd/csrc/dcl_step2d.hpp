@@ -14,6 +14,13 @@
 // phi is written once and not read back.  phi and kappa have the bits of the
 // separate SL and curvature kernels.
 //
+// With R = 4 a tile may also be wide: all 64 columns are its output, and the
+// column to either side is worked after them (32 nodes, one more round of one
+// wave; departures of a cell or more from these gather).  A wide tile takes
+// 7/6 of a narrow one's time, so it is the better one where it saves a column
+// of tiles of at most six, windows 64, 128, 192, 256 or 320 nodes wide above
+// all: 64 cells of 128 x 128 in FP32 19.2 us a step narrow, 15.5 wide.
+//
 // What it replaces read every stencil value with its own gather (about 20
 // vector loads per node, the texture path's limit) and phi again for the
 // curvature: 256 FP64 cells of edges 64 to 512 (1.9e7 nodes), tricubic RK2,
@@ -32,18 +39,43 @@ constexpr int S2_TX = 64, S2_TY = 4, S2_H = 3;  // threads of a block, phi0's ha
 
 template <int R>
 struct Step2 {
-  static constexpr int AY = S2_TY * R;                     // area rows
-  static constexpr int OX = S2_TX - 2, OY = AY - 2;        // output nodes
+  static constexpr bool WIDE = R == 4;                  // has wide tiles
+  static constexpr int AY = S2_TY * R;                  // area rows
+  static constexpr int AX = S2_TX + (WIDE ? 2 : 0);     // pitch of the new phi
+  static constexpr int OX = S2_TX - 2, OY = AY - 2;     // a narrow tile's output nodes
   static constexpr int PX = S2_TX + 2 * S2_H, PY = AY + 2 * S2_H;
-  static constexpr int VX = S2_TX + 3, VY = AY + 3;
+  static constexpr int VX = S2_TX + 3, VY = AY + 3;     // u ends a row earlier
   static constexpr int NT = S2_TX * S2_TY;
 };
 template <typename T, int R>
 struct Step2Lds {
   T phi[Step2<R>::PX * Step2<R>::PY];
-  T vel[2][Step2<R>::VX * Step2<R>::VY];
-  T out[Step2<R>::AY * S2_TX];
+  T u[Step2<R>::VX * (Step2<R>::VY - 1)], v[Step2<R>::VX * Step2<R>::VY];
+  T out[Step2<R>::AY * Step2<R>::AX];
 };
+// columns of a tile of a window this wide
+__host__ __device__ inline int step2d_cols(int nx, int rows) {
+  const bool wide = rows == 4 && 7 * ((nx + S2_TX - 1) / S2_TX) < 6 * ((nx + S2_TX - 3) / (S2_TX - 2));
+  return wide ? S2_TX : S2_TX - 2;
+}
+inline int64_t step2d_tiles(int nx, int ny, int rows) {
+  const int cols = step2d_cols(nx, rows), oy = S2_TY * rows - 2;
+  return (int64_t)((nx + cols - 1) / cols) * ((ny + oy - 1) / oy);
+}
+
+// Rows per thread, from the tiles there are with 4 and with 2: more rows stage
+// and recompute fewer halo values per node, fewer finish a small window sooner.
+// The lines lie where they cross, at 2.5 and 1.5 blocks per CU.  us per FP64
+// tricubic RK2 step with 1 / 2 / 4 rows, one window n x n: 128 3.2 / 4.3 /
+// 8.9, 256 4.2 / 4.5 / 6.4, 384 5.7 / 5.6 / 6.6, 512 8.1 / 6.9 / 8.5, 768 15.5
+// / 13.0 / 11.7, 1024 23.0 / 18.8 / 17.8; a batch of 128 x 128 cells: one 3.9 /
+// 5.2 / 8.2, 4 5.2 / 6.3 / 8.7, 8 7.4 / 6.9 / 8.8, 16 11.4 / 9.4 / 11.2, 32
+// 19.7 / 15.6 / 14.2, 64 35.3 / 28.4 / 20.7.  FP32 and the trilinear scheme
+// cross at about the same sizes.
+inline int step2d_rows(int64_t tiles4, int64_t tiles2, int cus) {
+  return 2 * tiles4 >= (int64_t)5 * cus ? 4 : 2 * tiles2 >= (int64_t)3 * cus ? 2 : 1;
+}
+
 // LDS reads through pointers of their own address space: where a branch reads
 // the same values from memory instead, the compiler would otherwise make one
 // flat load of the two
@@ -60,8 +92,8 @@ __device__ __forceinline__ T step2d_node(const T* __restrict__ phi0, const T* __
   const double Xd[2] = {(double)(P.w.px + i), (double)(P.w.py + j)};
   const int vo = (j - y0 + 1) * G::VX + (i - x0 + 1);
   T V[2];
-  V[0] = vmid(S.vel[0][vo], S.vel[0][vo + 1]);
-  V[1] = vmid(S.vel[1][vo], S.vel[1][vo + G::VX]);
+  V[0] = vmid(S.u[vo], S.u[vo + 1]);
+  V[1] = vmid(S.v[vo], S.v[vo + G::VX]);
   if (BT == DCL_RK2) {
     const double Xm[2] = {Xd[0] - (double)V[0] * P.ch[0], Xd[1] - (double)V[1] * P.ch[1]};
     int b0[3], b1[3];
@@ -69,14 +101,15 @@ __device__ __forceinline__ T step2d_node(const T* __restrict__ phi0, const T* __
     mac_split<T, 2>(P.v, Xm, b0, b1, f0, f1);
     // b0 <= b1 <= b0 + 1 along each axis
     const int lx = b0[0] - (x0 - 1), ly = b0[1] - (y0 - 1);
-    const bool in = lx >= 0 && b1[0] - (x0 - 1) <= G::VX - 2 && ly >= 0 && b1[1] - (y0 - 1) <= G::VY - 2;
+    const bool in = lx >= 0 && b1[0] - (x0 - 1) <= G::VX - 2 && ly >= 0 && ly <= G::VY - 3 &&
+                    b1[1] - (y0 - 1) <= G::VY - 2;
 #pragma unroll
     for (int c = 0; c < 2; ++c) {
       const int ix = c == 0 ? b1[0] : b0[0], iy = c == 1 ? b1[1] : b0[1];
       const T x1 = c == 0 ? f1[0] : f0[0], y1 = c == 1 ? f1[1] : f0[1];
       T a00, a10, a01, a11;
       if (in) {
-        const lds_cptr<T> q = (lds_cptr<T>)S.vel[c] + (iy - (y0 - 1)) * G::VX + (ix - (x0 - 1));
+        const lds_cptr<T> q = (lds_cptr<T>)(c == 0 ? S.u : S.v) + (iy - (y0 - 1)) * G::VX + (ix - (x0 - 1));
         a00 = q[0], a10 = q[1], a01 = q[G::VX], a11 = q[G::VX + 1];
       } else {
         const T* q = vel + (iy * nx + ix) * P.v.dof + P.v.udof + c * P.v.cs;
@@ -129,15 +162,16 @@ __device__ __forceinline__ T step2d_node(const T* __restrict__ phi0, const T* __
   }
 }
 
-// one tile: output nodes (ox .. ox + OX - 1, oy .. oy + OY - 1) clipped to
-// the window; kappa may be NULL (phi only).  Every thread of the block calls it; it ends on a barrier.
+// one tile: output nodes (ox .. ox + cols - 1, oy .. oy + OY - 1), cols as
+// step2d_cols says, clipped to the window; kappa may be NULL (phi only).  Every thread of the block calls it; it ends on a barrier.
 template <typename T, int INTERP, int BT, int R>
 __device__ __forceinline__ void step2d_tile(const T* __restrict__ phi0, T* __restrict__ phi, T* __restrict__ kappa,
                                             const T* __restrict__ vel, const SLP& P, T dx, T dy, const Curv2R<T>& cr, int ox,
-                                            int oy, Step2Lds<T, R>& S) {
+                                            int oy, int cols, Step2Lds<T, R>& S) {
   typedef Step2<R> G;
   const int nx = P.w.nx, ny = P.w.ny;
-  const int x0 = ox - 1, y0 = oy - 1;
+  const bool wide = G::WIDE && cols == S2_TX;
+  const int x0 = wide ? ox : ox - 1, y0 = oy - 1;
   const int tid = threadIdx.x + S2_TX * threadIdx.y;
   constexpr int NP = (G::PX * G::PY + G::NT - 1) / G::NT, NV = (G::VX * G::VY + G::NT - 1) / G::NT;
   T pv[NP], vv[NV][2];
@@ -163,32 +197,35 @@ __device__ __forceinline__ void step2d_tile(const T* __restrict__ phi0, T* __res
 #pragma unroll
   for (int q = 0; q < NV; ++q) {
     const int e = tid + q * G::NT;
-    if (e < G::VX * G::VY) {
-      S.vel[0][e] = vv[q][0];
-      S.vel[1][e] = vv[q][1];
-    }
+    if (e < G::VX * (G::VY - 1)) S.u[e] = vv[q][0];
+    if (e < G::VX * G::VY) S.v[e] = vv[q][1];
   }
   __syncthreads();
-  const int i = x0 + (int)threadIdx.x;
-#pragma unroll 1
-  for (int row = threadIdx.y; row < G::AY; row += S2_TY) {
-    const int j = y0 + row;
-    T v = S.phi[(row + S2_H) * G::PX + threadIdx.x + S2_H];
+  constexpr int C0 = G::WIDE ? 1 : 0;  // of the new phi: the column before the area
+  auto work = [&](int i, int j, int col, int row) {
+    T v = S.phi[(row + S2_H) * G::PX + col + S2_H];
     if (i >= 2 && i <= nx - 3 && j >= 2 && j <= ny - 3)
       v = step2d_node<T, INTERP, BT, R>(phi0, vel, P, S, x0, y0, i, j);
-    S.out[row * S2_TX + threadIdx.x] = v;
+    S.out[row * G::AX + col + C0] = v;
+  };
+  const int i = x0 + (int)threadIdx.x;
+#pragma unroll 1
+  for (int row = threadIdx.y; row < G::AY; row += S2_TY) work(i, y0 + row, threadIdx.x, row);
+  if (G::WIDE && wide && tid < 2 * G::AY) {
+    const int col = tid < G::AY ? -1 : S2_TX, row = tid % G::AY;
+    work(x0 + col, y0 + row, col, row);
   }
   __syncthreads();
-  if (threadIdx.x >= 1 && threadIdx.x <= G::OX && i < nx) {
+  if (i < nx && (wide || (threadIdx.x >= 1 && threadIdx.x <= G::OX))) {
 #pragma unroll
     for (int r = 0; r < R; ++r) {
       const int row = threadIdx.y + S2_TY * r, j = y0 + row;
       if (row < 1 || row > G::OY || j >= ny) continue;
-      phi[j * nx + i] = S.out[row * S2_TX + threadIdx.x];
+      const lds_cptr<T> p = (lds_cptr<T>)S.out + row * G::AX + threadIdx.x + C0;
+      phi[j * nx + i] = p[0];
       if (!kappa) continue;
       T k = T(0);
-      if (i >= 1 && i <= nx - 2 && j >= 1 && j <= ny - 2)
-        k = curv2d_recip_at<T>((lds_cptr<T>)S.out + row * S2_TX + threadIdx.x, S2_TX, dx, dy, cr);
+      if (i >= 1 && i <= nx - 2 && j >= 1 && j <= ny - 2) k = curv2d_recip_at<T>(p, G::AX, dx, dy, cr);
       kappa[j * nx + i] = k;
     }
   }

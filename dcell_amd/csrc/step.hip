@@ -22,34 +22,24 @@ __global__ __launch_bounds__(Step2<R>::NT) void step2d_k(const T* __restrict__ p
                                                          T* __restrict__ kappa, const T* __restrict__ vel, SLP P,
                                                          T dx, T dy, Curv2R<T> cr) {
   __shared__ Step2Lds<T, R> S;
-  step2d_tile<T, INTERP, BT, R>(phi0, phi, kappa, vel, P, dx, dy, cr, (int)blockIdx.x * Step2<R>::OX,
-                                (int)blockIdx.y * Step2<R>::OY, S);
+  const int cols = step2d_cols(P.w.nx, R);
+  step2d_tile<T, INTERP, BT, R>(phi0, phi, kappa, vel, P, dx, dy, cr, (int)blockIdx.x * cols,
+                                (int)blockIdx.y * Step2<R>::OY, cols, S);
 }
 
-template <int R>
-static dim3 step2d_grid(const KWin& w) {
-  return dim3((w.nx + Step2<R>::OX - 1) / Step2<R>::OX, (w.ny + Step2<R>::OY - 1) / Step2<R>::OY);
-}
-
-// Rows per thread: more rows stage and recompute fewer halo values per node,
-// fewer finish a small window sooner.  The lines lie where they cross, at 2.5
-// and 1.5 blocks per CU (us per FP64 tricubic RK2 step with 1 / 2 / 4 rows,
-// n x n: 128 3.2 / 4.3 / 8.9, 256 4.2 / 4.5 / 6.4, 384 5.7 / 5.6 / 6.6, 512
-// 8.1 / 6.9 / 8.5, 768 15.5 / 13.0 / 11.7, 1024 23.0 / 18.8 / 17.8; FP32 and
-// the trilinear scheme cross at the same sizes).
 template <typename T, int INTERP, int BT>
-static int step2d_launch(const T* phi0, T* phi, T* kappa, const T* vel, const SLP& P, T dx, T dy,
-                         hipStream_t s) {
+static int step2d_launch(const T* phi0, T* phi, T* kappa, const T* vel, const SLP& P, T dx, T dy, hipStream_t s) {
   const Curv2R<T> cr = curv2d_recips<T>(dx, dy);
-  // at least `halves` half blocks per CU
-  auto fills = [](dim3 g, int halves) { return 2 * (int64_t)g.x * g.y >= (int64_t)halves * device_cus(); };
-  const dim3 block(S2_TX, S2_TY);
-  if (fills(step2d_grid<4>(P.w), 5))
-    hipLaunchKernelGGL((step2d_k<T, INTERP, BT, 4>), step2d_grid<4>(P.w), block, 0, s, phi0, phi, kappa, vel, P, dx, dy, cr);
-  else if (fills(step2d_grid<2>(P.w), 3))
-    hipLaunchKernelGGL((step2d_k<T, INTERP, BT, 2>), step2d_grid<2>(P.w), block, 0, s, phi0, phi, kappa, vel, P, dx, dy, cr);
+  const int nx = P.w.nx, ny = P.w.ny;
+  const int rows = step2d_rows(step2d_tiles(nx, ny, 4), step2d_tiles(nx, ny, 2), device_cus());
+  const int cols = step2d_cols(nx, rows), oy = S2_TY * rows - 2;
+  const dim3 grid((nx + cols - 1) / cols, (ny + oy - 1) / oy), block(S2_TX, S2_TY);
+  if (rows == 4)
+    hipLaunchKernelGGL((step2d_k<T, INTERP, BT, 4>), grid, block, 0, s, phi0, phi, kappa, vel, P, dx, dy, cr);
+  else if (rows == 2)
+    hipLaunchKernelGGL((step2d_k<T, INTERP, BT, 2>), grid, block, 0, s, phi0, phi, kappa, vel, P, dx, dy, cr);
   else
-    hipLaunchKernelGGL((step2d_k<T, INTERP, BT, 1>), step2d_grid<1>(P.w), block, 0, s, phi0, phi, kappa, vel, P, dx, dy, cr);
+    hipLaunchKernelGGL((step2d_k<T, INTERP, BT, 1>), grid, block, 0, s, phi0, phi, kappa, vel, P, dx, dy, cr);
   DCL_LAUNCHED("step2d");
   return 0;
 }

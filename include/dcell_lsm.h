@@ -413,7 +413,8 @@ int dcl_batch_set_dt(dcl_batch batch, const double *dt);
  * shape (tile[] of dcl_batch_get_config), shape 6..11 = the curvature tiles
  * of shape - 6 with the SL step over 32 x 8 columns of the cell class's
  * z-chunk staged in an LDS ring; occupancy 0..2 -> 2, 4, 8 resident blocks
- * per CU.  2D batches use one tile whatever the shape. */
+ * per CU.  2D batches take a tile chosen from the number and the widths of
+ * their cells, whatever the shape (tile[]: cell 0's). */
 int dcl_batch_set_config(dcl_batch batch, int shape, int occupancy);
 int dcl_batch_get_config(dcl_batch batch, int *shape, int *occupancy, int32_t tile[3],
                          int *blocks);

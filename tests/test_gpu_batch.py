@@ -155,6 +155,36 @@ def test_batch_2d_matches_per_cell_oracle(dev, dtype, tp, tk, interp, bt):
     b.close()
 
 
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+@pytest.mark.parametrize("interp,bt", [("cubic", "rk2"), ("linear", "euler")])
+@pytest.mark.parametrize("edges,rows", [([128], 1), ([128] * 4, 1), ([64, 63, 65, 128, 126], 1), ([128] * 12, 2),
+                                        ([512, 500], 4), ([62, 63, 64, 65, 126, 127, 128, 129, 320] * 6, 4),
+                                        ([5, 6, 500, 640, 384, 192], 4)])
+def test_batch_2d_rows_by_the_tiles_there_are(dev, dtype, interp, bt, edges, rows):
+    """Few tiles take fewer rows per thread (tiles of 4 rows - 2), many four, in
+    62 or 64 columns; every cell gets the bits of its own dense step, also with
+    departures past the staged halo."""
+    rng = np.random.default_rng(len(edges))
+    wins = [D.GridWindow((c % 3, -1, 0), (n, max(5, n - c % 4), 1), (1.0 / n, 1.1 / n, 1.0))
+            for c, n in enumerate(edges)]
+    b = Batch(wins, dtype, interp, bt)
+    assert b.config()["tile"][1] == 4 * rows - 2
+    phi0, phi1, kap, vel = b.new_field(), b.new_field(), b.new_field(), b.new_field(2)
+    phi0.copy_(torch.from_numpy(rng.normal(size=b.nodes)))
+    vel.copy_(torch.from_numpy(rng.normal(size=2 * b.nodes)))
+    dts = [(0.4 if c % 2 else 1.1) / n for c, n in enumerate(edges)]
+    b.set_dt(dts)
+    for claim in (0, 4):
+        b.set_claim(claim)
+        phi1.fill_(7.0)
+        kap.fill_(7.0)
+        b.step(phi0, phi1, kap, vel)
+        for c, w in enumerate(wins):
+            p, k = D.levelset_step(b.cell(phi0, c), b.cell(vel, c, 2), w, dts[c], interp, bt)
+            assert torch.equal(b.cell(phi1, c), p) and torch.equal(b.cell(kap, c), k), (c, claim)
+    b.close()
+
+
 def _band_list(wins, phis, width, rng):
     """Nodes with |phi| < width of every cell as {x, y, z, cell} in a random
     order, plus each cell's (n, 3) band."""

@@ -296,10 +296,11 @@ def test_levelset_step_planes_equal_per_node(dev, dtype, dim):
 @pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
 @pytest.mark.parametrize("interp,bt", [("cubic", "rk2"), ("linear", "euler"), ("linear", "rk2")])
 @pytest.mark.parametrize("n,layout", [((5, 5), 2), ((62, 14), 2), ((63, 15), 1), ((61, 17), 3), ((125, 6), 2),
-                                      ((7, 300), 1), ((500, 430), 2), ((833, 801), 3)])
+                                      ((7, 300), 1), ((500, 430), 2), ((833, 801), 3), ((64, 9001), 2),
+                                      ((128, 4499), 1), ((127, 4500), 3), ((65, 4600), 2)])
 def test_levelset_step_2d_tiles(dev, dtype, interp, bt, n, layout):
     """The fused 2D step around its tile edges, at each number of rows per
-    thread, with every velocity layout (planes, (u, v), (p, u, v)) and
+    thread, in narrow and wide tiles, with every velocity layout (planes, (u, v), (p, u, v)) and
     departures on both sides of the staged halo: phi against the oracle and bit
     for bit the SL kernel's, kappa the curvature kernel's on that phi."""
     rng = np.random.default_rng(n[0] + n[1])
