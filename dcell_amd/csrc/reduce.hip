@@ -247,6 +247,7 @@ static size_t band_scratch_bytes(int64_t n) {
 // for it on each device, never the array's name.
 constexpr int64_t BAND_STATIC_MAX_NODES = (int64_t)1 << 28;
 constexpr size_t BAND_STATIC_BYTES = (4u << 20) + (64u << 10);
+constexpr size_t BAND_STATIC_TOTAL = 16;  // the total's bytes, before the rest
 static __device__ __align__(256) unsigned char band_static_scratch[BAND_STATIC_BYTES];
 
 constexpr int MAX_DEVICES = 64;
@@ -267,29 +268,33 @@ static int band_static_scratch_ptr(void** ptr) {
   return 0;
 }
 
+// the launches of a band compaction; the total goes to *total, which the
+// device writes (device or pinned memory)
 template <typename T>
-static int band_compact_t(const void* phi, const dcl_window* win, double width, dcl_icoor* out,
-                          int64_t cap, int64_t* count_out, void* sc, hipStream_t s) {
+static int band_launch_t(const void* phi, const dcl_window* win, double width, dcl_icoor* out, int64_t cap,
+                         unsigned long long* total, void* sc, hipStream_t s) {
   const int64_t n = win_nodes(*win);
   const int64_t nb = grid1d(n, RB);
   const int64_t ntiles = scan_tiles(nb);
-  HostResult total;
-  DCL_TRY(total.take());
   unsigned long long* sums = static_cast<unsigned long long*>(sc);
   unsigned* counts = reinterpret_cast<unsigned*>(sums + ntiles);
   const T* p = static_cast<const T*>(phi);
   hipLaunchKernelGGL((band_count_k<T>), dim3(nb), dim3(RB), 0, s, p, n, (T)width, counts);
   DCL_LAUNCHED("band_count");
-  const ScanArrays sa = {{counts, nullptr}, {sums, nullptr}, {total.as<unsigned long long>(), nullptr}};
+  const ScanArrays sa = {{counts, nullptr}, {sums, nullptr}, {total, nullptr}};
   DCL_TRY(scan_counts(sa, 1, nb, s));
   if (cap > 0) {
     hipLaunchKernelGGL((band_write_k<T>), dim3(nb), dim3(RB), 0, s, p, kwin(*win), n, (T)width, counts, sums,
                        out, cap);
     DCL_LAUNCHED("band_write");
   }
-  DCL_TRY(total.wait(s));
-  *count_out = (int64_t)*total.as<unsigned long long>();
   return 0;
+}
+
+static int band_launch(const void* phi, const dcl_window* win, double width, int precision, dcl_icoor* out,
+                       int64_t cap, unsigned long long* total, void* sc, hipStream_t s) {
+  return precision == DCL_F64 ? band_launch_t<double>(phi, win, width, out, cap, total, sc, s)
+                              : band_launch_t<float>(phi, win, width, out, cap, total, sc, s);
 }
 
 static int check_band_compact(const void* phi, const dcl_window* win, int precision, const dcl_icoor* band_out,
@@ -309,8 +314,12 @@ extern "C" int dcl_band_compact(const void* phi, const dcl_window* win, double w
   hipStream_t s = as_stream(stream);
   void* sc = nullptr;
   DCL_TRY(scratch(band_scratch_bytes(win_nodes(*win)), &sc));
-  if (precision == DCL_F64) return band_compact_t<double>(phi, win, width, band_out, capacity, count_out, sc, s);
-  return band_compact_t<float>(phi, win, width, band_out, capacity, count_out, sc, s);
+  HostResult total;
+  DCL_TRY(total.take());
+  DCL_TRY(band_launch(phi, win, width, precision, band_out, capacity, total.as<unsigned long long>(), sc, s));
+  DCL_TRY(total.wait(s));
+  *count_out = (int64_t)*total.as<unsigned long long>();
+  return 0;
 }
 
 extern "C" int dcl_band_compact_static(const void* phi, const dcl_window* win, double width, int precision,
@@ -318,7 +327,7 @@ extern "C" int dcl_band_compact_static(const void* phi, const dcl_window* win, d
                                        void* stream) {
   DCL_TRY(check_band_compact(phi, win, precision, band_out, capacity, count_out));
   const int64_t n = win_nodes(*win);
-  if (n > BAND_STATIC_MAX_NODES || band_scratch_bytes(n) > BAND_STATIC_BYTES)
+  if (n > BAND_STATIC_MAX_NODES || BAND_STATIC_TOTAL + band_scratch_bytes(n) > BAND_STATIC_BYTES)
     return set_error(DCL_ERR_ARG_SIZ,
                      "window of %lld nodes: the allocation-free band compaction takes windows of up to "
                      "%lld nodes (its static scratch holds %zu bytes)",
@@ -326,8 +335,16 @@ extern "C" int dcl_band_compact_static(const void* phi, const dcl_window* win, d
   void* sc = nullptr;
   DCL_TRY(band_static_scratch_ptr(&sc));
   hipStream_t s = as_stream(stream);
-  if (precision == DCL_F64) return band_compact_t<double>(phi, win, width, band_out, capacity, count_out, sc, s);
-  return band_compact_t<float>(phi, win, width, band_out, capacity, count_out, sc, s);
+  // The total lies in the array too and is copied back: a HostResult's pinned
+  // word would be allocated by the process's first call.
+  unsigned long long* total = static_cast<unsigned long long*>(sc);
+  DCL_TRY(band_launch(phi, win, width, precision, band_out, capacity, total,
+                      static_cast<char*>(sc) + BAND_STATIC_TOTAL, s));
+  unsigned long long tot = 0;
+  DCL_HIP(hipMemcpyAsync(&tot, total, sizeof(tot), hipMemcpyDeviceToHost, s));
+  DCL_HIP(hipStreamSynchronize(s));
+  *count_out = (int64_t)tot;
+  return 0;
 }
 
 extern "C" int dcl_interface_metrics(const void* phi, const void* kappa, const dcl_window* win,
