@@ -52,8 +52,10 @@ int scratch(size_t bytes, void** ptr);
 // 22.6 us with a copy to the caller's pageable word, which is staged and
 // awaited by itself.  The words are one of HR_SLOTS of the process, allocated
 // together by the first call that needs one (all in use: an allocation of the
-// call's own); they are given back once the stream has been waited for, and
-// stay taken where that failed, since a kernel may still write them.
+// call's own).  A call gives them back when it returns, also with an error
+// between take() and wait(): the destructor then waits for the stream.  They
+// stay taken only where the stream cannot be waited for, since a kernel may
+// still write them.
 class HostResult {
  public:
   static constexpr int HR_SLOTS = 64, HR_BYTES = 64;
@@ -61,14 +63,15 @@ class HostResult {
   ~HostResult();
   HostResult(const HostResult&) = delete;
   HostResult& operator=(const HostResult&) = delete;
-  int take();
-  int wait(hipStream_t s);
+  int take(hipStream_t s);
+  int wait();
   template <typename V>
   V* as() const { return static_cast<V*>(p_); }
 
  private:
   void* p_ = nullptr;
   int slot_ = -1;
+  hipStream_t s_ = nullptr;
   bool waited_ = false;
 };
 

@@ -729,7 +729,7 @@ static int irregular_t(const void* phi, const dcl_window* win, const dcl_icoor* 
   DCL_TRY(scratch(tasks_off + sizeof(IrrTask) * (size_t)nb, &sc));
   char* base = static_cast<char*>(sc);
   HostResult records;
-  DCL_TRY(records.take());
+  DCL_TRY(records.take(s));
   unsigned long long* sums = reinterpret_cast<unsigned long long*>(base + sums_off);
   unsigned* counts = reinterpret_cast<unsigned*>(base + counts_off);
   const ScanArrays sa = {{counts, reinterpret_cast<unsigned*>(base + counts_off + counts_bytes)},
@@ -741,7 +741,7 @@ static int irregular_t(const void* phi, const dcl_window* win, const dcl_icoor* 
   const int rc = win->n.z >= 2 ? irr_launch<T, 3>(p, w, band, nb, sa, tasks, out, cap, s)
                                : irr_launch<T, 2>(p, w, band, nb, sa, tasks, out, cap, s);
   if (rc) return rc;
-  DCL_TRY(records.wait(s));
+  DCL_TRY(records.wait());
   *count_out = (int64_t)*records.as<unsigned long long>();
   return 0;
 }

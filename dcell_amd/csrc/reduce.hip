@@ -214,9 +214,9 @@ extern "C" int dcl_max_velocity(const dcl_velocity* vel, const void* nodes, int6
   void* sc = nullptr;
   DCL_TRY(scratch(sizeof(double) * nb, &sc));
   double* part = static_cast<double*>(sc);
-  HostResult res;
-  DCL_TRY(res.take());
   hipStream_t s = as_stream(stream);
+  HostResult res;
+  DCL_TRY(res.take(s));
   const char* nd = static_cast<const char*>(nodes);
 #define DCL_MV(T, D)                                                                        \
   hipLaunchKernelGGL((maxvel_k<T, D>), dim3(nb), dim3(RB), 0, s, static_cast<const T*>(vel->data), \
@@ -230,7 +230,7 @@ extern "C" int dcl_max_velocity(const dcl_velocity* vel, const void* nodes, int6
   DCL_LAUNCHED("maxvel");
   hipLaunchKernelGGL((fold_partials_k<1>), dim3(1), dim3(RB), 0, s, part, nb, res.as<double>(), 1, 0, 0, 0);
   DCL_LAUNCHED("fold_partials");
-  DCL_TRY(res.wait(s));
+  DCL_TRY(res.wait());
   *max_out = res.as<double>()[0];
   return 0;
 }
@@ -315,9 +315,9 @@ extern "C" int dcl_band_compact(const void* phi, const dcl_window* win, double w
   void* sc = nullptr;
   DCL_TRY(scratch(band_scratch_bytes(win_nodes(*win)), &sc));
   HostResult total;
-  DCL_TRY(total.take());
+  DCL_TRY(total.take(s));
   DCL_TRY(band_launch(phi, win, width, precision, band_out, capacity, total.as<unsigned long long>(), sc, s));
-  DCL_TRY(total.wait(s));
+  DCL_TRY(total.wait());
   *count_out = (int64_t)*total.as<unsigned long long>();
   return 0;
 }
@@ -359,9 +359,9 @@ extern "C" int dcl_interface_metrics(const void* phi, const void* kappa, const d
   void* sc = nullptr;
   DCL_TRY(scratch(sizeof(double) * 3 * nb, &sc));
   double* part = static_cast<double*>(sc);
-  HostResult res;
-  DCL_TRY(res.take());
   hipStream_t s = as_stream(stream);
+  HostResult res;
+  DCL_TRY(res.take(s));
   const KWin w = kwin(*win);
 #define DCL_MT(T, D)                                                                             \
   hipLaunchKernelGGL((metrics_k<T, D>), dim3(nb), dim3(RB), 0, s, static_cast<const T*>(phi),       \
@@ -375,7 +375,7 @@ extern "C" int dcl_interface_metrics(const void* phi, const void* kappa, const d
   DCL_LAUNCHED("interface_metrics");
   hipLaunchKernelGGL((fold_partials_k<3>), dim3(1), dim3(RB), 0, s, part, nb, res.as<double>(), 0, 0, 0, 0);
   DCL_LAUNCHED("fold_partials");
-  DCL_TRY(res.wait(s));
+  DCL_TRY(res.wait());
   const double* r = res.as<double>();
   out[0] = r[0];
   out[1] = r[1];
@@ -398,9 +398,9 @@ extern "C" int dcl_error_norms(const void* a, int prec_a, const void* b, int pre
   void* sc = nullptr;
   DCL_TRY(scratch(sizeof(double) * 3 * nb, &sc));
   double* part = static_cast<double*>(sc);
-  HostResult res;
-  DCL_TRY(res.take());
   hipStream_t s = as_stream(stream);
+  HostResult res;
+  DCL_TRY(res.take(s));
 #define DCL_NM(TA, TB)                                                                         \
   hipLaunchKernelGGL((norms_k<TA, TB>), dim3(nb), dim3(RB), 0, s, static_cast<const TA*>(a),       \
                      static_cast<const TB*>(b), n, part)
@@ -412,7 +412,7 @@ extern "C" int dcl_error_norms(const void* a, int prec_a, const void* b, int pre
   DCL_LAUNCHED("error_norms");
   hipLaunchKernelGGL((fold_partials_k<3>), dim3(1), dim3(RB), 0, s, part, nb, res.as<double>(), 1, 0, 1, 0);
   DCL_LAUNCHED("fold_partials");
-  DCL_TRY(res.wait(s));
+  DCL_TRY(res.wait());
   for (int k = 0; k < 3; ++k) out[k] = res.as<double>()[k];
   return 0;
 }

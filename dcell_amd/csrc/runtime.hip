@@ -105,7 +105,8 @@ static std::mutex g_hr_mu;
 static char* g_hr;
 static uint64_t g_hr_used;  // one bit a slot
 
-int HostResult::take() {
+int HostResult::take(hipStream_t s) {
+  s_ = s;
   static_assert(HR_SLOTS == 64, "one bit of g_hr_used a slot");
   {
     std::lock_guard<std::mutex> lock(g_hr_mu);
@@ -125,14 +126,18 @@ int HostResult::take() {
   return 0;
 }
 
-int HostResult::wait(hipStream_t s) {
-  DCL_HIP(hipStreamSynchronize(s));
+int HostResult::wait() {
+  DCL_HIP(hipStreamSynchronize(s_));
   waited_ = true;
   return 0;
 }
 
 HostResult::~HostResult() {
-  if (!p_ || !waited_) return;
+  if (!p_) return;
+  if (!waited_ && hipStreamSynchronize(s_) != hipSuccess) {
+    (void)hipGetLastError();
+    return;
+  }
   if (slot_ < 0) {
     (void)hipHostFree(p_);
     return;

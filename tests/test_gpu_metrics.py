@@ -37,8 +37,9 @@ def test_max_velocity_with_irregular_node_stride(dev, dim):
 
 @pytest.mark.parametrize("threads", [3, 80])
 def test_host_results_of_concurrent_calls(dev, threads):
-    """Each thread's calls return its own result, also with more calls under
-    way than the process keeps host words for."""
+    """Each thread's calls return its own result, from few threads and from more
+    than the process keeps host words for (how many calls are under way at once
+    is up to the scheduler; test_host_results.py counts the words)."""
     n = 24
     win = D.GridWindow((0, 0, 0), (n, n, n), (1.0, 1.0, 1.0))
     vel = random_velocity(n, 3, np.random.default_rng(3), 1.0)

@@ -62,3 +62,36 @@ ts = [threading.Thread(target=lambda: band(static=True, count=C.c_int64())) for 
 [t.join() for t in ts]
 assert get("stub_allocs") == get("stub_frees") == 0, (get("stub_allocs"), get("stub_frees"))
 """)
+
+
+def test_result_words_come_back(stub):
+    """The 64 pinned words are one allocation; a call that fails between taking
+    its word and waiting for the stream gives it back; with all of them taken a
+    call allocates its own and frees it; a word whose stream cannot be waited
+    for stays taken."""
+    run(stub, """
+assert band() == 0, lib.dcl_last_error()
+assert get("stub_host_allocs") == 1
+put("stub_fail_launch", 1)
+for _ in range(200):
+    assert band() != 0
+put("stub_fail_launch", 0)
+assert band() == 0 and get("stub_host_allocs") == 1
+# 70 calls under way at once: none returns before the last waits for its stream
+stub.stub_reset_hold(70)
+rc = []
+ts = [threading.Thread(target=lambda: rc.append(band(count=C.c_int64()))) for _ in range(70)]
+[t.start() for t in ts]
+[t.join() for t in ts]
+stub.stub_reset_hold(0)
+assert rc == [0] * 70
+assert get("stub_host_allocs") == 1 + 6 and get("stub_host_frees") == 6
+assert band() == 0 and get("stub_host_allocs") == 7
+put("stub_fail_sync", 1)
+for _ in range(64):
+    assert band() != 0
+assert get("stub_host_allocs") == 7
+put("stub_fail_sync", 0)
+assert band() == 0
+assert get("stub_host_allocs") == 8 and get("stub_host_frees") == 7
+""")
