@@ -276,7 +276,11 @@ __device__ __forceinline__ bool ri_pop_round(const RiHeap& H, const RiLane& t, c
   RiEntry e;
   e.v = right ? r.v : l.v;
   e.key = right ? r.key : l.key;
-  const bool stop = bubble.v - e.v <= 0;
+  // An infinite bubble (a tentative value that overflowed) stops above an
+  // infinite or a missing child, where the difference is NaN; the reference
+  // goes on past an infinite one, which moves infinite entries only, and these
+  // are never accepted.
+  const bool stop = !(bubble.v - e.v > 0);
   const uint64_t sm = __builtin_amdgcn_ballot_w64(stop);
   // the node is its parent's smaller child
   const uint64_t cm =

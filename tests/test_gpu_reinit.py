@@ -103,6 +103,38 @@ def test_reinit_heap_levels_and_faces(dev, n):
     _check(phi, win, recs, dphi, band)
 
 
+def test_reinit_infinite_tentative_values(dev):
+    """Tentative values that overflow to infinity fill a heap deeper than its
+    part in LDS while ordinary nodes are accepted: the last entry, moved down at
+    each pop, is infinite where the heap has no child.  A node between P along
+    x and Q along y gets (2 P + 2 Q + sqrt((2 P + 2 Q)^2 - 8 (P^2 + Q^2))) / 4,
+    whose first square rounds past the largest number for these two and the
+    second sum does not."""
+    P, Q = np.nextafter(2.0 ** 510, 0), 2.0 ** 510
+    B = -2.0 * P - 2.0 * Q
+    with np.errstate(over="ignore"):
+        assert np.isinf(np.float64(B) * B) and np.isfinite(8.0 * (-1.0 + P * P + Q * Q))
+    nx, ny = 260, 300
+    win = D.GridWindow((0, 0, 0), (nx, ny, 1), (1.0, 1.0, 1.0))
+    y, x = np.meshgrid(np.arange(ny), np.arange(nx), indexing="ij")
+    low = x == 5                                        # an ordinary front, pushed first
+    high = (x >= 20) & ((x + y) % 2 == 0)
+    phi = np.ones((ny, nx))
+    at = np.concatenate([np.argwhere(low), np.argwhere(high)])
+    recs = np.zeros(len(at), dtype=M.IRREGULAR_DTYPE)
+    recs["pos"][:, 0], recs["pos"][:, 1] = at[:, 1], at[:, 0]
+    recs["axis"] = recs["shift"] = -1
+    recs["sign_center"] = 1
+    recs["op"][:, 0] = np.where(at[:, 1] == 5, 0.25, np.where(at[:, 0] % 2 == 0, P, Q))
+    drecs = torch.from_numpy(recs.view(np.uint8).reshape(-1).copy()).to("cuda:0")
+    dphi = to_dev(phi)
+    (band,) = M.reinitialize([(dphi, win, drecs, len(recs))], 6.0, 2.0 ** 600, heap_capacity=8 * len(recs))
+    ref_phi, ref_band = O.reinitialize(phi, owin(win), recs, 6.0, 2.0 ** 600)
+    assert len(ref_band) > len(recs) + 5 * ny           # the front was marched
+    assert to_np(dphi).tobytes() == ref_phi.tobytes()
+    np.testing.assert_array_equal(to_np(band), ref_band)
+
+
 def test_reinit_empty_and_heap_error(dev):
     n = 20
     win = D.GridWindow((0, 0, 0), (n, n, n), (1.0, 1.0, 1.0))
