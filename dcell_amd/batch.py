@@ -2,7 +2,7 @@
 
 The cells' windows (all 3D or all 2D) are packed back to back in one phi
 buffer, one kappa buffer and one velocity buffer; ``Batch.step`` runs the SL
-step and the curvature of every cell in two persistent launches,
+step and the curvature of every cell in two persistent launches (one in 2D),
 ``Batch.band_step`` the same at listed nodes only (band mode),
 ``Batch.autotune`` picks the tile shape, the occupancy and each size class's
 z-chunk by timing them, and ``Batch.graph`` records a step as a hipGraph for

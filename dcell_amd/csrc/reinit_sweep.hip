@@ -41,7 +41,6 @@
 #include <math.h>
 #include <string.h>
 
-#include "dcl_buf.hpp"
 #include "dcl_host.hpp"
 #include "dcl_reinit.hpp"
 
@@ -50,11 +49,14 @@ namespace dcl {
 constexpr int RS_B = 256;
 constexpr double RS_TOL = 1e-9;  // settled: no node moves by more than band_width * RS_TOL
 constexpr int RS_OUT = 3;        // the mask of a stencil node outside the window
-constexpr int RS_CH = 1024;      // nodes per chunk of the mark scan (four per thread)
+constexpr int RS_CH = 1024;      // nodes per chunk of the mark scan (one wave, 16 per lane)
 constexpr int RS_STAGE = 3072;   // list entries a block gathers before publishing them
 // blocks of the mark scan: each publishes its entries with an atomic on one
-// counter, and fewer leave waves idle (a 256^3 step with 512, 1024, 2048 and
-// 4096: 1.64, 1.60, 1.78 and 2.05 ms)
+// counter, and fewer leave waves idle.  ms with 512, 1024, 2048 and 4096: a
+// 256^3 step 1.64, 1.60, 1.78, 2.05; level sets of edges 32 to 48, 4 of them
+// 0.81, 0.76, 0.79, 0.79, 64 of them 2.75, 2.73, 3.02, 3.30; 256 of 32 to 64
+// 11.8, 10.5, 10.1, 10.4; 1000 of 24 to 32 21.3, 19.9, 19.2, 19.3; 64 of 96
+// 10.5, 9.2, 8.5, 8.9.
 constexpr int RS_NEED_GRID = 1024;
 constexpr int RS_GRID = 4096;       // blocks of the update, each taking listed nodes in turn
 constexpr int RS_GROUP = 4;         // sweeps queued between looks at the count of level sets still sweeping
@@ -502,9 +504,9 @@ __device__ __forceinline__ bool rs_update_node(const RsCell& c, RsState* __restr
 }
 
 template <int DIM>
-__global__ __launch_bounds__(RS_B) __attribute__((amdgpu_waves_per_eu(3, 8))) void rs_update_k(const RsCell* __restrict__ cells, RsState* __restrict__ st,
-                                                    const int2* __restrict__ nlist, const int* __restrict__ ncount,
-                                                    unsigned long long* __restrict__ parts, int nparts, int pstride) {
+__global__ __launch_bounds__(RS_B) __attribute__((amdgpu_waves_per_eu(3, 8))) void rs_update_k(
+    const RsCell* __restrict__ cells, RsState* __restrict__ st, const int2* __restrict__ nlist,
+    const int* __restrict__ ncount, unsigned long long* __restrict__ parts, int nparts, int pstride) {
   const int n = *ncount;
   for (int e0 = blockIdx.x * RS_B; e0 < n; e0 += gridDim.x * RS_B) {
     const int e = e0 + threadIdx.x;

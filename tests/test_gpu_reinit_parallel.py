@@ -8,9 +8,9 @@ window's faces, a 2D circle, a batch of level sets of different sizes that
 settle after different numbers of sweeps, a 2D batch holding a level set
 without records, an empty record list, a band capacity below the band's
 length (the count still whole, the prefix written), too few sweeps allowed
-and a batch mixing 2D and 3D (errors), and a 294M-node window (the
-large-window load path) checked against the closed-form distance to a
-plane."""
+and a batch mixing 2D and 3D (errors), and a 294M-node window (node indices
+and byte offsets past 2^28 and 2^31) checked against the closed-form distance
+to a plane."""
 import numpy as np
 import pytest
 import torch
@@ -184,11 +184,11 @@ def test_parallel_every_node_marked(dev):
 
 
 def test_parallel_large_window_flat_path(dev):
-    """A window of 2^28 nodes or more (700 x 700 x 600) takes the large-window
-    path (64-bit pointer loads instead of 32-bit buffer offsets).  phi = 3 x
-    the distance to the plane z = 300.3, so the answer is closed-form: the
-    exact distance on every node within band_width (1e-12, each z-plane
-    uniform), +-PHI_INF elsewhere, and the band is exactly those nodes."""
+    """A window of more than 2^28 nodes (700 x 700 x 600), whose byte offsets
+    pass 2^31: the same kernels at large indices.  phi = 3 x the distance to
+    the plane z = 300.3, so the answer is closed-form: the exact distance on
+    every node within band_width (1e-12, each z-plane uniform), +-PHI_INF
+    elsewhere, and the band is exactly those nodes."""
     nx, ny, nz = 700, 700, 600
     assert nx * ny * nz >= 1 << 28
     win = D.GridWindow((0, 0, 0), (nx, ny, nz), (1.0, 1.0, 1.0))
