@@ -26,7 +26,7 @@
 // curvature: 256 FP64 cells of edges 64 to 512 (1.9e7 nodes), tricubic RK2,
 // 406 -> 251 us per step (1.8 -> 3.0 TB/s of the 40 bytes per node); a 128 x
 // 128 step replayed from a graph 4.7 -> 3.2 us, one launch instead of two.
-// The FP64 tile (R = 4) takes 40.9 KB of LDS and 113 registers, four blocks
+// The FP64 tile (R = 4) takes 40.6 KB of LDS and 113 registers, four blocks
 // per CU by either; the arithmetic is about 60% of its time.
 #pragma once
 
